@@ -112,7 +112,7 @@ __device__ __forceinline__ int tile_of_block(int bid, int tiles_x, int tiles_y) 
 // differently: on config 5's near-singular conics, whose terms cancel, that
 // moved alphas across the 1/255 cutoff.
 __device__ __forceinline__ float4 scale_conic(const float4 con) {
-    return make_float4(-0.5f * con.x, -con.y, -0.5f * con.z, 0.f);
+    return make_float4(-0.5f * con.x, -con.y, -0.5f * con.z, con.w);
 }
 
 // The exponent of the splat at offset (dx, dy) from the staged conic.
@@ -154,18 +154,32 @@ __device__ __forceinline__ float rect_min_q(float mux, float muy, float a, float
     return best;
 }
 
+// One batch entry's record in LDS, 48 bytes: the walks read it with one
+// address as two full 16-byte words and one 4-byte word. With the nine floats
+// in three float4s of which three lanes each were used, the compiler read 12
+// bytes of each, and a 12-byte LDS read takes about twice a 16-byte one's
+// cycles here: the LDS was active 29.4M cycles in the forward's walk at 300k
+// Gaussians and 800x800, now 13.5M (and one address register an entry instead
+// of three).
+struct __align__(16) LdsRec {
+    float4 geo;       // u, v, opacity, red
+    float4 con;       // scaled conic (see scale_conic), green
+    float blue;
+    int32_t id;
+    uint32_t live;    // bit w: wave w may be touched
+    float pad;
+};
+static_assert(sizeof(LdsRec) == 48, "three 16-byte words");
+
 // LDS of one workgroup; MAXW bounds the waves per tile (4 up to 16x16).
 template <int MAXW>
 struct Stage {
-    float4 geo[kBatch];       // u, v, opacity, unused
-    float4 con[kBatch];       // conic a, b, c, unused
-    float4 col[kBatch];       // r, g, b, unused
-    int32_t id[kBatch];
-    uint32_t live[kBatch];    // bit w: wave w may be touched
-    uint16_t list[MAXW][kBatch];
-    float4 rect[MAXW];        // x_lo, x_hi, y_lo, y_hi of pixel centres
+    LdsRec rec[kBatch];
+    uint8_t list[MAXW][kBatch];   // each wave's live entries
+    float4 rect[MAXW];            // x_lo, x_hi, y_lo, y_hi of pixel centres
     int32_t flag[MAXW];
 };
+static_assert(kBatch <= 256, "list entries are bytes");
 
 constexpr int kGradSlots = 10;   // colour 3, moments 5, sum dg, |d uv|
 
@@ -283,35 +297,36 @@ __device__ __forceinline__ float reduce18(const float a[9], const float b[9], in
 // ten slots of one entry together, which then fall in distinct LDS banks.
 constexpr int kGradStride = kBatch + 1;
 
-template <int MAXW>
+template <int MAXW, int SLOTS>
 struct StageBwd : Stage<MAXW> {
-    float grad[kGradSlots][kGradStride];   // per batch entry, summed over waves
+    float grad[SLOTS][kGradStride];   // per batch entry, summed over waves
 };
 
 // One list entry's record, gathered from the per-Gaussian arrays.
 struct Rec {
-    float4 geo;   // u, v, opacity
-    float4 con;   // conic a, b, c
-    float4 col;   // r, g, b
+    float4 geo;   // u, v, opacity, red
+    float4 con;   // conic a, b, c, green
+    float blue;
     int32_t id;
 };
 
 __device__ __forceinline__ Rec gather_rec(const RasterArgs &A, int g) {
     Rec r;
     r.id = g;
-    r.geo = make_float4(A.uv[2 * g], A.uv[2 * g + 1], A.opac[g], 0.f);
-    r.con = make_float4(A.conic[3 * g], A.conic[3 * g + 1], A.conic[3 * g + 2], 0.f);
-    r.col = make_float4(A.color[3 * g], A.color[3 * g + 1], A.color[3 * g + 2], 0.f);
+    r.geo = make_float4(A.uv[2 * g], A.uv[2 * g + 1], A.opac[g], A.color[3 * g]);
+    r.con = make_float4(A.conic[3 * g], A.conic[3 * g + 1], A.conic[3 * g + 2],
+                        A.color[3 * g + 1]);
+    r.blue = A.color[3 * g + 2];
     return r;
 }
 
 // Writes entry t's record to LDS with its per-wave cull bits.
 template <class S_>
 __device__ __forceinline__ void put_rec(S_ &S, int t, const Rec &r, int nwaves) {
-    S.geo[t] = r.geo;
-    S.con[t] = scale_conic(r.con);
-    S.col[t] = r.col;
-    S.id[t] = r.id;
+    S.rec[t].geo = r.geo;
+    S.rec[t].con = scale_conic(r.con);
+    S.rec[t].blue = r.blue;
+    S.rec[t].id = r.id;
     const float thr = 2.0f * __logf(fmaxf(255.0f * r.geo.z, 1.0f));
     const float thr_m = thr * 1.0001f + 1e-4f;
     uint32_t m = 0;
@@ -323,7 +338,7 @@ __device__ __forceinline__ void put_rec(S_ &S, int t, const Rec &r, int nwaves) 
             rect_min_q(r.geo.x, r.geo.y, ca, r.con.y, cc, ia, ic, q.x, q.y, q.z, q.w) < thr_m)
             m |= 1u << w;
     }
-    S.live[t] = m;
+    S.rec[t].live = m;
 }
 
 template <class S_>
@@ -352,9 +367,9 @@ __device__ __forceinline__ int compact_live(S_ &S, int n, int lim, int wave, int
     int cnt = 0;
     for (int c = 0; c < n; c += 64) {
         const int j = c + lane;
-        const bool bit = j < n && j < lim && ((S.live[j] >> wave) & 1u);
+        const bool bit = j < n && j < lim && ((S.rec[j].live >> wave) & 1u);
         const uint64_t m = ballot(bit);
-        if (bit) S.list[wave][cnt + rank_in(m)] = (uint16_t)j;
+        if (bit) S.list[wave][cnt + rank_in(m)] = (uint8_t)j;
         cnt += __popcll(m);
     }
     wave_sync_lds();
@@ -556,7 +571,10 @@ __global__ __launch_bounds__(MAXW * 64) __attribute__((amdgpu_waves_per_eu(8))) 
     publish_rect(S, inimg, fx, fy, wave, lane);
 
     const int start = A.offsets[tile_id], end = A.offsets[tile_id + 1];
-    float T = 1.0f, cr = 0.f, cg = 0.f, cb = 0.f, acc = 0.f;
+    float T = 1.0f, cr = 0.f, cg = 0.f, cb = 0.f;
+    // A pixel is done once T < t_min after a splat; T starts at 1, so with a
+    // threshold above 1 the first splat ends it.
+    const float t_min = A.t_min > 1.0f ? 1.0f : A.t_min;
     int stop = start;
     bool done = !inimg;
     // Checkpoints: pixel slot inside the tile, next unit to record.
@@ -590,16 +608,17 @@ __global__ __launch_bounds__(MAXW * 64) __attribute__((amdgpu_waves_per_eu(8))) 
             for (int k = 0; k < cnt; k += U) {
                 if ((k & 63) == 0 && k) lreg = S.list[wave][k + lane];
                 int jj[U];
-                float4 gg[U], kk[U], cc[U];
+                float4 gg[U], kk[U];
+                float bb[U];
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     // Past the end, the round's last real entry again (masked
                     // below); a scalar min keeps the lane index in scalar registers.
                     const int ku = min(k + u, cnt - 1);
                     jj[u] = __builtin_amdgcn_readlane(lreg, ku & 63);
-                    gg[u] = S.geo[jj[u]];
-                    kk[u] = S.con[jj[u]];
-                    cc[u] = S.col[jj[u]];
+                    gg[u] = S.rec[jj[u]].geo;
+                    kk[u] = S.rec[jj[u]].con;
+                    bb[u] = S.rec[jj[u]].blue;
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
@@ -609,15 +628,20 @@ __global__ __launch_bounds__(MAXW * 64) __attribute__((amdgpu_waves_per_eu(8))) 
                                               gg[u].z * __expf(power));
                     const bool live = (u == 0 || k + u < cnt) && !done && power <= 0.0f &&
                                       alpha >= kAlphaMin;
-                    const float w = live ? alpha * T : 0.0f;
-                    cr = fmaf(w, cc[u].x, cr);
-                    cg = fmaf(w, cc[u].y, cg);
-                    cb = fmaf(w, cc[u].z, cb);
-                    acc += w;
-                    const float Tn = T * (1.0f - alpha);
-                    T = live ? Tn : T;
+                    // One select: with alpha 0 the weight is 0 and T keeps
+                    // its value, T (1 - 0) = T. The walk's vector issue sets
+                    // its pace (81% of the cycles), so every instruction an
+                    // entry counts: this, the coverage taken from T and the
+                    // record's layout took the forward from 118 to 104 us at
+                    // 1M Gaussians and 800x800, 136 to 118 at 3.6M crowded.
+                    const float al = live ? alpha : 0.0f;
+                    const float w = al * T;
+                    cr = fmaf(w, gg[u].w, cr);
+                    cg = fmaf(w, kk[u].w, cg);
+                    cb = fmaf(w, bb[u], cb);
+                    T *= 1.0f - al;
                     stop = live ? base + jj[u] + 1 : stop;
-                    done = done || (live && Tn < A.t_min);
+                    done = done || T < t_min;
                 }
                 if (ballot(!done) == 0) break;
             }
@@ -649,6 +673,8 @@ __global__ __launch_bounds__(MAXW * 64) __attribute__((amdgpu_waves_per_eu(8))) 
     zero_fill();
     if (!inimg) return;
     const int64_t o = (int64_t)py * A.W + px;
+    // The weights alpha T sum to 1 - T.
+    const float acc = 1.0f - T;
     if (A.has_bg) {
         // Rounded as the separate torch ops of metal_backend.py's blend
         // (rgb + (1 - alpha).clamp_min(0) * bg): no fused multiply-add.
@@ -682,7 +708,8 @@ template <int MAXW, bool ABS, bool PIPE>
 __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs A,
                                                                const RasterGrads G,
                                                                const ChunkPlan P) {
-    __shared__ StageBwd<MAXW> S;
+    constexpr int kSlots = ABS ? 10 : 9;
+    __shared__ StageBwd<MAXW, kSlots> S;
     // Without a plan a workgroup takes a whole tile; with one, one chunk.
     int tile_id, chunk = 0, tile_start, tile_end;
     if (P.ckpt) {
@@ -762,7 +789,7 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
 
     // One list entry's update of the pixel; v gets the pixel's share of the
     // entry's sums (zeros where it is not active). Returns whether it is.
-    auto update = [&](const int i, const float4 geo, const float4 con, const float4 col,
+    auto update = [&](const int i, const float4 geo, const float4 con, const float blue,
                       float v[kGradSlots]) {
         const float dx = fx - geo.x, dy = fy - geo.y;
         const float power = splat_power(dx, dy, con);
@@ -777,14 +804,14 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
         // T / (1 - alpha) with a 1-ulp reciprocal; the forward's rounding of
         // T (1 - alpha) already makes the recovery approximate.
         // alpha <= 0.999 (fminf returns 0.999 for a NaN product too), so
-        // 1 - alpha >= 0.001 needs no lower clamp.
-        const float om = 1.0f - alpha;
-        const float iom = __builtin_amdgcn_rcpf(om);
-        const float gc = fmaf(gb, col.z, fmaf(gg, col.y, fmaf(gr, col.x, ga)));
+        // 1 - alpha >= 0.001 needs no lower clamp. An inactive lane takes
+        // alpha 0: 1 / (1 - 0) is 1 and T and Gs keep their values.
+        const float al = active ? alpha : 0.0f;
+        const float iom = __builtin_amdgcn_rcpf(1.0f - al);
+        const float gc = fmaf(gb, blue, fmaf(gg, con.w, fmaf(gr, geo.w, ga)));
         const float dal = (T * gc - Gs) * iom;
-        const float Tn = T * iom;
-        const float w = active ? alpha * Tn : 0.0f;
-        T = active ? Tn : T;
+        T *= iom;
+        const float w = al * T;
         Gs = fmaf(w, gc, Gs);
         // Past the 0.999 clamp alpha no longer depends on the splat.
         const float dg = active && alpha_raw <= kAlphaMax ? dal * gauss : 0.0f;
@@ -811,10 +838,10 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
 
     // One list entry: the pixel's update and the wave's sums into S.grad.
     auto entry = [&](const int j, const int i, const float4 geo, const float4 con,
-                     const float4 col) {
+                     const float blue) {
         float v[kGradSlots];
         // With no lane active the update leaves T and Gs as they were.
-        if (ballot(update(i, geo, con, col, v)) == 0) return;
+        if (ballot(update(i, geo, con, blue, v)) == 0) return;
         // Sums over the wave of v[0..9], deposited into S.grad[.][j] with
         // four lanes per LDS atomic (see reduce10_to_rows).
         float q0, q1, q2;
@@ -836,9 +863,9 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
     // Two consecutive entries (back to front: a, then b), their eighteen
     // sums in one reduction and one LDS atomic per sum (without |d uv|).
     const int slot18 = reduce18_slot(lane);
-    auto entry2 = [&](const int ja, const float4 geo_a, const float4 con_a, const float4 col_a,
+    auto entry2 = [&](const int ja, const float4 geo_a, const float4 con_a, const float col_a,
                       const int jb, const float4 geo_b, const float4 con_b,
-                      const float4 col_b, const int base) {
+                      const float col_b, const int base) {
         float va[kGradSlots], vb[kGradSlots];
         const bool act_a = update(base + ja, geo_a, con_a, col_a, va);
         const bool act_b = update(base + jb, geo_b, con_b, col_b, vb);
@@ -851,11 +878,11 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
     // in place in S.grad: d_uv = op (a Sx + b Sy, b Sx + c Sy), d_conic =
     // -op (Sxx / 2, Sxy, Syy / 2), d_op = S1, d_col, and |d_uv| = op Sabs.
     auto take = [&](const int e) {
-        float s[kGradSlots];
+        float s[kSlots];
 #pragma unroll
-        for (int q = 0; q < kGradSlots; ++q) s[q] = S.grad[q][e];
-        const float op = S.geo[e].z;
-        const float3 con = raw_conic(S.con[e]);
+        for (int q = 0; q < kSlots; ++q) s[q] = S.grad[q][e];
+        const float op = S.rec[e].geo.z;
+        const float3 con = raw_conic(S.rec[e].con);
         S.grad[0][e] = op * fmaf(con.x, s[3], con.y * s[4]);
         S.grad[1][e] = op * fmaf(con.y, s[3], con.z * s[4]);
         S.grad[2][e] = -0.5f * op * s[5];
@@ -865,16 +892,16 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
         S.grad[6][e] = s[0];
         S.grad[7][e] = s[1];
         S.grad[8][e] = s[2];
-        S.grad[9][e] = op * s[9];
+        if (ABS) S.grad[kSlots - 1][e] = op * s[kSlots - 1];
     };
     // The workgroup's atomics, (entry, slot)-major: consecutive lanes hit
     // consecutive slots of one record.
     auto flush = [&](const int n) {
-        constexpr int V = ABS ? 10 : 9;
+        constexpr int V = kSlots;
         for (int idx = (int)threadIdx.x; idx < V * n; idx += (int)blockDim.x) {
             const int e = idx / V, v = idx - V * e;
             const float val = S.grad[v][e];
-            if (val != 0.f) unsafeAtomicAdd(G.rec + (int64_t)kRecFloats * S.id[e] + v, val);
+            if (val != 0.f) unsafeAtomicAdd(G.rec + (int64_t)kRecFloats * S.rec[e].id + v, val);
         }
     };
 
@@ -901,7 +928,7 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
         } else {
             stage_batch(S, A, base, n, nwaves);
         }
-        for (int q = t; q < kGradSlots * kGradStride; q += blockDim.x) (&S.grad[0][0])[q] = 0.f;
+        for (int q = t; q < kSlots * kGradStride; q += blockDim.x) (&S.grad[0][0])[q] = 0.f;
         __syncthreads();
         if (PIPE) {
             // Batches below the first are full.
@@ -920,23 +947,25 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
             int k = cnt - 1;
             int lreg = S.list[wave][(k & ~63) + lane];
             int ja = __builtin_amdgcn_readlane(lreg, k & 63), jc;
-            float4 geo_a = S.geo[ja], con_a = S.con[ja], col_a = S.col[ja];
-            float4 geo_c, con_c, col_c;
+            float4 geo_a = S.rec[ja].geo, con_a = S.rec[ja].con;
+            float col_a = S.rec[ja].blue;
+            float4 geo_c, con_c;
+            float col_c;
             // Entry k - 1 into (jx, x) and entry max(k - 2, 0) into (jy, y).
-            auto read2 = [&](int &jx, float4 &gx, float4 &kx, float4 &cx, int &jy, float4 &gy,
-                             float4 &ky, float4 &cy) {
+            auto read2 = [&](int &jx, float4 &gx, float4 &kx, float &cx, int &jy, float4 &gy,
+                             float4 &ky, float &cy) {
                 const int kb = k - 1;
                 if ((kb & 63) == 63) lreg = S.list[wave][(kb & ~63) + lane];
                 jx = __builtin_amdgcn_readlane(lreg, kb & 63);
-                gx = S.geo[jx];
-                kx = S.con[jx];
-                cx = S.col[jx];
+                gx = S.rec[jx].geo;
+                kx = S.rec[jx].con;
+                cx = S.rec[jx].blue;
                 const int kc = max(k - 2, 0);
                 if ((kc & 63) == 63) lreg = S.list[wave][(kc & ~63) + lane];
                 jy = __builtin_amdgcn_readlane(lreg, kc & 63);
-                gy = S.geo[jy];
-                ky = S.con[jy];
-                cy = S.col[jy];
+                gy = S.rec[jy].geo;
+                ky = S.rec[jy].con;
+                cy = S.rec[jy].blue;
             };
             for (;;) {
                 if (k == 0) {
@@ -945,7 +974,8 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
                 }
                 {
                     int jb;
-                    float4 geo_b, con_b, col_b;
+                    float4 geo_b, con_b;
+                    float col_b;
                     read2(jb, geo_b, con_b, col_b, jc, geo_c, con_c, col_c);
                     entry2(ja, geo_a, con_a, col_a, jb, geo_b, con_b, col_b, base);
                 }
@@ -957,7 +987,8 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
                 }
                 {
                     int jd;
-                    float4 geo_d, con_d, col_d;
+                    float4 geo_d, con_d;
+                    float col_d;
                     read2(jd, geo_d, con_d, col_d, ja, geo_a, con_a, col_a);
                     entry2(jc, geo_c, con_c, col_c, jd, geo_d, con_d, col_d, base);
                 }
@@ -968,21 +999,23 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
             int k = cnt - 1;
             int lreg = S.list[wave][(k & ~63) + lane];
             int ja = __builtin_amdgcn_readlane(lreg, k & 63);
-            float4 geo_a = S.geo[ja], con_a = S.con[ja], col_a = S.col[ja];
+            float4 geo_a = S.rec[ja].geo, con_a = S.rec[ja].con;
+            float col_a = S.rec[ja].blue;
             for (;;) {
                 // Entry k - 1 (or k again at the end) into the b registers.
                 const int kb = max(k - 1, 0);
                 if ((kb & 63) == 63) lreg = S.list[wave][(kb & ~63) + lane];
                 const int jb = __builtin_amdgcn_readlane(lreg, kb & 63);
-                const float4 geo_b = S.geo[jb], con_b = S.con[jb], col_b = S.col[jb];
+                const float4 geo_b = S.rec[jb].geo, con_b = S.rec[jb].con;
+                const float col_b = S.rec[jb].blue;
                 entry(ja, base + ja, geo_a, con_a, col_a);
                 if (--k < 0) break;
                 const int kc = max(k - 1, 0);
                 if ((kc & 63) == 63) lreg = S.list[wave][(kc & ~63) + lane];
                 ja = __builtin_amdgcn_readlane(lreg, kc & 63);
-                geo_a = S.geo[ja];
-                con_a = S.con[ja];
-                col_a = S.col[ja];
+                geo_a = S.rec[ja].geo;
+                con_a = S.rec[ja].con;
+                col_a = S.rec[ja].blue;
                 entry(jb, base + jb, geo_b, con_b, col_b);
                 if (--k < 0) break;
             }

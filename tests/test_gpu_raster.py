@@ -110,6 +110,22 @@ def test_forward_matches_contract(dev, tile, t_min):
     assert (np_(stop) == r[3])[ok].all(), "stop indices differ"
 
 
+@pytest.mark.parametrize("t_min", [0.3, 1.0, 2.0])
+def test_forward_stops_at_large_thresholds(dev, t_min):
+    """From a threshold of 1 up a pixel holds its first splat alone; the
+    coverage is 1 - T. Bars as above."""
+    W, H, tile = 100, 63, 16
+    args = prepare(600, 17, W, H, tile, dev)
+    rgb, alpha, T, stop, _ = gpu_forward(args, W, H, tile, t_min)
+    r = raster_ref.forward(*[np_(a) for a in args[:6]], W, H, tile, t_min)
+    ok = ~r[4]
+    assert np.abs(np_(rgb) - r[0])[ok].max() < 1e-4
+    assert np.abs(np_(alpha) - r[1])[ok].max() < 1e-4
+    assert (np_(stop) == r[3])[ok].all(), "stop indices differ"
+    # 1 - T is rounded once from T, which lies in [0, 1].
+    assert np.array_equal(np_(alpha), np.float32(1.0) - np_(T))
+
+
 @pytest.mark.parametrize("chunked", [True, False])
 @pytest.mark.parametrize("tile", [8, 12, 16, 32])
 def test_backward_matches_contract(dev, tile, chunked):
