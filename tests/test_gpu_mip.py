@@ -233,6 +233,36 @@ def test_compute_3d_filter_matches_oracle(dev, n_views):
     assert bad.sum() <= max(2, n // 2000), f"{bad.sum()} mismatches, worst {rel.max():.2e}"
 
 
+@pytest.mark.parametrize("n,n_views", [(1, 1), (64, 3), (65, 4), (1000, 257), (196_607, 9),
+                                       (196_608, 9)])
+def test_compute_3d_filter_without_divisions_is_bit_exact(dev, n, n_views):
+    """A near plane below the depth clamp makes the kernel decide every pair by
+    the reference's divisions. With every point in front of the other near
+    plane too, the two results must be the same bits. Frames are off centre
+    and cut through the points, so many pairs lie near a bound."""
+    from metal_gauss_amd import compute_3d_filter
+
+    g = np.random.default_rng(n + n_views)
+    means = (g.uniform(-1.0, 1.0, (n, 3))).astype(np.float32)
+    # Points on a bound's own grid: u lands on or within an ulp of it.
+    means[::7] = np.round(means[::7] * 8) / 8
+    views = []
+    for i in range(n_views):
+        W, H = int(g.integers(64, 900)), int(g.integers(64, 900))
+        f = float(g.uniform(300, 1200))
+        K = np.array([[f, 0, W * g.uniform(0.2, 0.8)], [0, f, H / 2], [0, 0, 1.0]])
+        eye = g.standard_normal(3)
+        vm = _look_at(eye / np.linalg.norm(eye) * 4.0) if i % 3 else np.eye(4)
+        if i % 3 == 0:
+            vm[2, 3] = 4.0
+        views.append(_View(torch.from_numpy(K.astype(np.float32)),
+                           torch.from_numpy(vm.astype(np.float32)), W, H))
+    m = torch.from_numpy(means).to(dev)
+    fast = compute_3d_filter(m, views, near=0.2)
+    divided = compute_3d_filter(m, views, near=0.0)
+    assert torch.equal(fast, divided)
+
+
 def test_compute_3d_filter_reference_cases(dev):
     """tests/test_mipfilter.py:108-144 on the GPU kernel."""
     from metal_gauss_amd import compute_3d_filter
