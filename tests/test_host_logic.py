@@ -204,3 +204,38 @@ def test_fused_adam_refused_step_keeps_the_epilogue_bookkeeping():
         with pytest.raises(RuntimeError, match="already applied"):
             opt.step()
     assert opt._epilogue_applied == {id(p): p}
+
+
+def _loop_view_records(views, margin):
+    """The records of mipfilter.py:45-66, one view at a time."""
+    rows, focal = [], 0.0
+    for v in views:
+        vm, K = v.viewmat.detach().double(), v.K.detach().double()
+        H, W = v.image.shape[:2]
+        fx, fy, cx, cy = float(K[0, 0]), float(K[1, 1]), float(K[0, 2]), float(K[1, 2])
+        rows.append(vm[:3, :3].reshape(-1).tolist() + vm[:3, 3].tolist() +
+                    [fx, fy, cx, cy, -margin * W, (1.0 + margin) * W, -margin * H,
+                     (1.0 + margin) * H])
+        focal = max(focal, fx, fy)
+    return (torch.tensor(rows, dtype=torch.float32) if rows else torch.zeros(0, 20)), focal
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("n_views", [0, 1, 7])
+def test_view_records_equal_the_per_view_loop(n_views, mixed):
+    from types import SimpleNamespace
+
+    from metal_gauss_amd.mipfilter import _view_records
+
+    g = torch.Generator().manual_seed(n_views)
+    views = []
+    for i in range(n_views):
+        K = torch.rand(3, 3, generator=g) * 1000.0
+        vm = torch.randn(4, 4, generator=g).requires_grad_(i == 2)
+        if mixed and i == 1:
+            K, vm = K.double(), vm.detach()[:3]
+        views.append(SimpleNamespace(K=K, viewmat=vm, image=torch.empty(97 + i, 203 + i, 3)))
+    for margin in (0.15, 0.0):
+        rec, focal = _view_records(iter(views), 0.2, margin)
+        want, want_focal = _loop_view_records(views, margin)
+        assert torch.equal(rec, want) and focal == want_focal
