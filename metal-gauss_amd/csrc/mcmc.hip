@@ -22,9 +22,9 @@
 // counted with integer atomics. Copies and source updates are separate
 // launches: every copy reads its source before any source is rewritten.
 //
-// The per-row work runs one wave per touched row over the concatenated
-// columns of all parameter and optimizer-state tensors (59 + 118 floats per
-// row for a 3DGS parameter set), so each tensor row is a contiguous span.
+// The draws are one dense list of (destination, source) pairs, and the row
+// work is spread over its elements tensor by tensor (59 parameter and 118
+// state floats per row for a 3DGS parameter set), see mcmc_rows_kernel.
 #include "mg_common.h"
 
 namespace mg {
@@ -199,81 +199,108 @@ __global__ __launch_bounds__(kScanThreads) void mcmc_reduce_kernel(const WeightA
     }
 }
 
-// Pass 2 (one workgroup): exclusive scan of the block sums of both arrays in
-// place, and the totals.
+// Pass 2 (one workgroup): exclusive scan of the block sums of both arrays and
+// of the dead counts in place, and the totals.
 __global__ __launch_bounds__(1024) void mcmc_block_scan_kernel(double *blk_w, double *blk_o,
-                                                               const int64_t *blk_dead,
+                                                               int64_t *blk_dead,
                                                                const int32_t *blk_bad, int nblk,
                                                                McmcTotals *tot) {
     __shared__ double s_w[16], s_o[16];
-    __shared__ double c_w, c_o;
-    __shared__ int64_t s_dead;
-    __shared__ int32_t s_bad, s_pos;
+    __shared__ int64_t s_d[16];
+    __shared__ int32_t s_f[16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (threadIdx.x == 0) { c_w = 0.0; c_o = 0.0; s_dead = 0; s_bad = 0; s_pos = 0; }
-    __syncthreads();
+    // Every thread carries the totals so far.
+    double c_w = 0.0, c_o = 0.0;
+    int64_t c_d = 0;
+    int32_t flags = 0;
     for (int b0 = 0; b0 < nblk; b0 += 1024) {
         const int b = b0 + (int)threadIdx.x;
-        const double vw = b < nblk ? blk_w[b] : 0.0, vo = b < nblk ? blk_o[b] : 0.0;
+        const bool in = b < nblk;
+        const double vw = in ? blk_w[b] : 0.0, vo = in ? blk_o[b] : 0.0;
+        const int64_t vd = in ? blk_dead[b] : 0;
+        const int32_t vf = in ? blk_bad[b] : 0;
         double iw = vw, io = vo;
+        int64_t id = vd;
         for (int o = 1; o < 64; o <<= 1) {
             const double tw = __shfl_up(iw, o, 64), to = __shfl_up(io, o, 64);
-            if (lane >= o) { iw += tw; io += to; }
+            const int64_t td = __shfl_up(id, o, 64);
+            if (lane >= o) { iw += tw; io += to; id += td; }
         }
-        if (lane == 63) { s_w[wave] = iw; s_o[wave] = io; }
-        if (b < nblk) {
-            atomicAdd((unsigned long long *)&s_dead, (unsigned long long)blk_dead[b]);
-            if (blk_bad[b] & 1) s_bad = 1;
-            if (blk_bad[b] & 2) s_pos = 1;
-        }
+        const int32_t wf = (ballot((vf & 1) != 0) != 0 ? 1 : 0) |
+                           (ballot((vf & 2) != 0) != 0 ? 2 : 0);
+        if (lane == 63) { s_w[wave] = iw; s_o[wave] = io; s_d[wave] = id; s_f[wave] = wf; }
         __syncthreads();
         double pw = c_w, po = c_o;
-        for (int w = 0; w < wave; ++w) { pw += s_w[w]; po += s_o[w]; }
-        if (b < nblk) { blk_w[b] = pw + iw - vw; blk_o[b] = po + io - vo; }
-        __syncthreads();
-        if (threadIdx.x == 1023) { c_w = pw + iw; c_o = po + io; }
+        int64_t pd = c_d;
+        for (int w = 0; w < wave; ++w) { pw += s_w[w]; po += s_o[w]; pd += s_d[w]; }
+        if (in) {
+            blk_w[b] = pw + iw - vw;
+            blk_o[b] = po + io - vo;
+            blk_dead[b] = pd + id - vd;
+        }
+        // The last wave's running sums, in the same order of additions.
+        for (int w = wave; w < 15; ++w) { pw += s_w[w]; po += s_o[w]; pd += s_d[w]; }
+        c_w = pw + s_w[15];
+        c_o = po + s_o[15];
+        c_d = pd + s_d[15];
+        for (int w = 0; w < 16; ++w) flags |= s_f[w];
         __syncthreads();
     }
     if (threadIdx.x == 0) {
         tot->sum_w = c_w;
         tot->sum_o = c_o;
-        tot->n_dead = s_dead;
-        tot->nonfinite = s_bad;
-        tot->has_pos = s_pos;
+        tot->n_dead = c_d;
+        tot->nonfinite = flags & 1;
+        tot->has_pos = flags >> 1;
     }
 }
 
 // Pass 3: inclusive CDF of the chosen weights (block offset + in-block scan,
-// rows in the same order as pass 1).
+// rows in the same order as pass 1); under relocate also the list of dead
+// rows, in row order.
 __global__ __launch_bounds__(kScanThreads) void mcmc_cdf_kernel(const WeightArgs W,
                                                                 const double *blk_off,
-                                                                double *cdf) {
+                                                                const int64_t *dead_off,
+                                                                double *cdf, int32_t *dst) {
     __shared__ double s_w[kScanThreads / 64];
+    __shared__ int32_t s_n[kScanThreads / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t base = (int64_t)blockIdx.x * kScanBlock;
     double carry = blk_off[blockIdx.x];
+    int64_t dcarry = W.grow ? 0 : dead_off[blockIdx.x];
     for (int k = 0; k < kScanItems; ++k) {
         const int64_t i = base + (int64_t)k * kScanThreads + threadIdx.x;
         double v = 0.0;
+        bool dead = false;
         if (i < W.n) {
             double w, o;
-            bool dead, b, ps;
+            bool b, ps;
             row_weights(W, i, w, o, dead, b, ps);
             v = W.use_opac ? o : w;
         }
+        const uint64_t dm = ballot(dead);
         double inc = v;
         for (int o = 1; o < 64; o <<= 1) {
             const double t = __shfl_up(inc, o, 64);
             if (lane >= o) inc += t;
         }
         __syncthreads();
-        if (lane == 63) s_w[wave] = inc;
+        if (lane == 63) {
+            s_w[wave] = inc;
+            s_n[wave] = __popcll(dm);
+        }
         __syncthreads();
         double pre = carry;
         for (int w = 0; w < wave; ++w) pre += s_w[w];
         if (i < W.n) cdf[i] = pre + inc;
         for (int w = wave; w < kScanThreads / 64; ++w) pre += s_w[w];
         carry = pre;   // carry + this round's total, the same in every thread
+        if (!W.grow) {
+            int64_t at = dcarry + rank_in(dm);
+            for (int w = 0; w < wave; ++w) at += s_n[w];
+            if (dead) dst[at] = (int32_t)i;
+            for (int w = 0; w < kScanThreads / 64; ++w) dcarry += s_n[w];
+        }
     }
 }
 
@@ -306,51 +333,35 @@ __device__ __forceinline__ int64_t cdf_search(const WeightArgs &W, const double 
     return lo;
 }
 
-// Draws. Relocate: one per dead row i < n (counter i); the source is kept at
-// the row itself, src[i], and rows that are not dead get -1. Grow: one per
-// j < n_draw (counter j), for destination dst0 + j, source src[j].
+// Draws, one thread each: draw j's source goes to src[j], with the top bit set
+// for the draw that counts its source first. Relocate draws for destination
+// dst[j] (the dead rows) with that row as the counter, grow for destination
+// dst0 + j with counter j.
+constexpr uint32_t kFirst = 0x80000000u;
+
 struct DrawArgs {
     WeightArgs W;
     const double *cdf;
-    int64_t n_draw;      // grow only
+    int64_t n_draw;
     uint64_t k0, k1;
-    int32_t *src, *counts;
+    const int32_t *dst;       // relocate only
+    const McmcTotals *tot;    // relocate only: dst holds tot->n_dead rows
+    uint32_t *src;
+    int32_t *counts;
 };
 
 __global__ __launch_bounds__(256) void mcmc_draw_kernel(const DrawArgs D) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (j >= (D.tot ? min(D.n_draw, D.tot->n_dead) : D.n_draw)) return;
     const int64_t n = D.W.n;
     const double last = D.cdf[n - 1];
-    if (D.W.grow) {
-        if (i >= D.n_draw) return;
-    } else {
-        if (i >= n) return;
-        double w, o;
-        bool dead, b, ps;
-        row_weights(D.W, i, w, o, dead, b, ps);
-        if (!dead) {
-            D.src[i] = -1;
-            return;
-        }
-    }
+    const int64_t i = D.W.grow ? j : (int64_t)D.dst[j];
     const U64x4 r = philox4x64((uint64_t)i, 0, 0, 0, D.k0, D.k1);
     const int64_t s = cdf_search(D.W, D.cdf, n, u01d(r.x[0]) * last);
-    D.src[i] = (int32_t)s;
-    atomicAdd(&D.counts[s], 1);
+    D.src[j] = (uint32_t)s | (atomicAdd(&D.counts[s], 1) == 0 ? kFirst : 0u);
 }
 
 // ------------------------------------------------------ per-row updates
-struct RowTensors {
-    float *p[kMaxTensors];
-    int32_t width[kMaxTensors];   // floats per row
-    int32_t kind[kMaxTensors];    // 0 copied param, 1 log-scales, 2 logit, 3 zeroed state
-    int32_t col0[kMaxTensors];    // first column of each tensor in a row's concatenation
-    int32_t cols;                 // columns of all tensors
-    int32_t src_col0[kMaxTensors];   // the same over the tensors a source update touches
-    int32_t src_cols;             // (kinds 1-3; copied tensors sit below column 0)
-    int32_t count;
-};
-
 constexpr int kMaxMult = 51;      // mcmc.py:33
 
 // The N-way split of opacity o: the new opacity, its logit and the log of
@@ -368,79 +379,124 @@ __device__ __forceinline__ float multiplicity(const int32_t *counts, int64_t s, 
     return (float)c;
 }
 
-enum RowMode { kRelocateCopies = 0, kGrowCopies = 1, kSources = 2 };
+// The row work as tasks, one or two per tensor, each over the list's rows:
+// copies (destination <- source; the logit <- the split's, the log scales plus
+// its log ratio), and the optimizer state of destinations and of sources <- 0.
+// A workgroup takes a run of rows of one task, its threads the run's elements
+// in order: reads and writes of a row are contiguous, and every element's
+// loads are independent. One wave per row over all tensors' columns, as
+// before, waited for the row's source, its count and opacity, the split and
+// the row in turn: 96 us for the copies and as much for the sources of 100k
+// draws of 177 floats from 900k rows, now 97 + 10 us. What is left is memory:
+// clearing the sources' state is 1.1M scattered pieces of rows (43 us), the
+// copies' source rows 0.6M (29 us), the destinations' state one span a tensor
+// (25 us). The copies read the sources' logits and log scales, which a second
+// launch then updates.
+enum RowOp { kCopy = 0, kCopyScales = 1, kCopyLogit = 2, kZeroDst = 3, kZeroSrc = 4 };
 
-// One workgroup per `chunk` candidates (a power of two up to 256, chosen so
-// that a workgroup holds about one selected row per wave): the selected ones
-// (relocate: dead rows; grow: every draw; sources: rows drawn at least once)
-// are compacted in LDS, then each wave takes one selected row at a time and
-// spreads the row's columns, across every tensor, over its 64 lanes. The
-// tensor table sits in LDS, where each lane finds its column's tensor.
-//   copies:  destination <- source, logit <- split logit, log-scales <-
-//            source's + log ratio, optimizer state <- 0;
-//   sources: logit <- split logit, log-scales += log ratio, state <- 0.
-template <int MODE>
-__global__ __launch_bounds__(256) void mcmc_rows_kernel(const RowTensors R, const int32_t *src,
-                                                        const int32_t *counts,
-                                                        const float *logit, int64_t n_cand,
-                                                        int64_t dst0, int grow, int chunk) {
-    __shared__ float *s_p[kMaxTensors];
-    __shared__ int32_t s_w[kMaxTensors], s_kind[kMaxTensors], s_col0[kMaxTensors];
-    __shared__ int32_t s_list[256];
-    __shared__ int32_t s_cnt;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid < R.count) {
-        s_p[tid] = R.p[tid];
-        s_w[tid] = R.width[tid];
-        s_kind[tid] = R.kind[tid];
-        s_col0[tid] = MODE == kSources ? R.src_col0[tid] : R.col0[tid];
-    }
-    if (tid == 0) s_cnt = 0;
-    __syncthreads();
-    const int64_t c0 = (int64_t)blockIdx.x * chunk;
-    bool sel = false;
-    if (tid < chunk && c0 + tid < n_cand) {
-        if (MODE == kRelocateCopies) sel = src[c0 + tid] >= 0;
-        else if (MODE == kGrowCopies) sel = true;
-        else sel = counts[c0 + tid] > 0;
-    }
-    const uint64_t m = ballot(sel);
-    int base = 0;
-    if (lane == 0 && m) base = atomicAdd(&s_cnt, __popcll(m));
-    base = __shfl(base, 0, 64);
-    if (sel) s_list[base + rank_in(m)] = tid;
-    __syncthreads();
-    const int cnt = s_cnt;
-    const int cols = MODE == kSources ? R.src_cols : R.cols;
-    const int count = R.count;
-    for (int e = wave; e < cnt; e += 4) {
-        const int64_t ci = c0 + s_list[e];
-        int64_t d = 0, sr;
-        if (MODE == kRelocateCopies) { d = ci; sr = src[ci]; }
-        else if (MODE == kGrowCopies) { d = dst0 + ci; sr = src[ci]; }
-        else sr = ci;
-        float logit_new, log_ratio;
-        split(sigmoidf(logit[sr]), multiplicity(counts, sr, grow), logit_new, log_ratio);
-        int t = 0;
-        for (int col = lane; col < cols; col += 64) {
-            while (t + 1 < count && s_col0[t + 1] <= col) ++t;
-            float *p = s_p[t];
-            const int64_t w = s_w[t];
-            const int k = col - s_col0[t], kind = s_kind[t];
-            if (MODE == kSources) {
-                if (kind == 3) p[sr * w + k] = 0.0f;
-                else if (kind == 2) p[sr * w + k] = logit_new;
-                else p[sr * w + k] += log_ratio;
-            } else {
-                float v;
-                if (kind == 3) v = 0.0f;
-                else if (kind == 2) v = logit_new;
-                else if (kind == 1) v = p[sr * w + k] + log_ratio;
-                else v = p[sr * w + k];
-                p[d * w + k] = v;
+constexpr int kMaxTasks = 2 * kMaxTensors;
+constexpr int kRowElems = 2048;   // elements of a workgroup's run (one row at least)
+
+struct RowTasks {
+    float *p[kMaxTasks];
+    int32_t width[kMaxTasks], op[kMaxTasks];
+    int32_t rows[kMaxTasks];         // rows of a workgroup's run
+    uint32_t block0[kMaxTasks + 1];  // first workgroup of each task
+    int32_t count;
+    // The source update's tensors.
+    float *logit, *log_scales;
+    int32_t scales_width;
+};
+
+struct RowList {
+    const int32_t *dst;     // destinations, or null: dst0 + j
+    const uint32_t *src;
+    const int32_t *counts;
+    const float *logit;     // the candidates' opacity logits
+    int64_t n, dst0;
+    int32_t grow;
+    const McmcTotals *tot;  // relocate only
+
+    __device__ __forceinline__ int64_t rows() const { return tot ? min(n, tot->n_dead) : n; }
+};
+
+__global__ __launch_bounds__(256) void mcmc_rows_kernel(const RowTasks R, const RowList L) {
+    // The workgroup's task: the tasks that end at or before it, counted by the
+    // lanes of a wave (a scan of the table was a chain of scalar loads).
+    static_assert(kMaxTasks == 64, "a lane per task");
+    const int lane = threadIdx.x & 63;
+    const uint32_t end = R.block0[lane + 1];
+    const int t = (int)__popcll(ballot(lane < R.count && end <= blockIdx.x));
+    const int w = R.width[t], op = R.op[t], rows = R.rows[t];
+    float *const p = R.p[t];
+    const int64_t j0 = (int64_t)(blockIdx.x - R.block0[t]) * rows;
+    const int64_t n_el = min((int64_t)rows, L.rows() - j0) * w;
+    const bool one = rows == 1;
+    // e / w by a multiplication, exact for e < 2^12 and w up to there.
+    const uint32_t inv = (uint32_t)((1u << 24) + (uint32_t)w - 1u) / (uint32_t)w;
+    // kRowElems elements at a time, kRowPer a thread: their list entries are
+    // requested together, then their values, then stored.
+    constexpr int kRowPer = kRowElems / 256;
+    for (int64_t e0 = threadIdx.x; e0 < n_el; e0 += kRowElems) {
+        int64_t j[kRowPer], k[kRowPer];
+        uint32_t q[kRowPer];
+        float v[kRowPer];
+        bool on[kRowPer];
+#pragma unroll
+        for (int i = 0; i < kRowPer; ++i) {
+            // Past the run, its last element again, not stored.
+            const int64_t e = e0 + 256 * i, ec = min(e, n_el - 1);
+            const int jj = one ? 0 : (int)(((uint64_t)ec * inv) >> 24);
+            j[i] = j0 + jj;
+            k[i] = ec - (int64_t)jj * w;
+            on[i] = e < n_el;
+        }
+        if (op != kZeroDst) {
+#pragma unroll
+            for (int i = 0; i < kRowPer; ++i) q[i] = L.src[j[i]];
+            if (op == kZeroSrc) {
+#pragma unroll
+                for (int i = 0; i < kRowPer; ++i)
+                    if (on[i] && (q[i] & kFirst)) p[(int64_t)(q[i] & ~kFirst) * w + k[i]] = 0.0f;
+                continue;
             }
         }
+        // Destination rows.
+#pragma unroll
+        for (int i = 0; i < kRowPer; ++i) j[i] = L.dst ? (int64_t)L.dst[j[i]] : L.dst0 + j[i];
+#pragma unroll
+        for (int i = 0; i < kRowPer; ++i) v[i] = 0.0f;
+        if (op == kCopy || op == kCopyScales) {
+#pragma unroll
+            for (int i = 0; i < kRowPer; ++i) v[i] = p[(int64_t)(q[i] & ~kFirst) * w + k[i]];
+        }
+        if (op == kCopyScales || op == kCopyLogit) {
+#pragma unroll
+            for (int i = 0; i < kRowPer; ++i) {
+                const int64_t s = q[i] & ~kFirst;
+                float logit_new, log_ratio;
+                split(sigmoidf(L.logit[s]), multiplicity(L.counts, s, L.grow), logit_new,
+                      log_ratio);
+                v[i] = op == kCopyLogit ? logit_new : v[i] + log_ratio;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kRowPer; ++i)
+            if (on[i]) p[j[i] * w + k[i]] = v[i];
     }
+}
+
+// The sources' own split, one thread per distinct source.
+__global__ __launch_bounds__(256) void mcmc_sources_kernel(const RowTasks R, const RowList L) {
+    const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (j >= L.rows()) return;
+    const uint32_t q = L.src[j];
+    if (!(q & kFirst)) return;
+    const int64_t s = q & ~kFirst;
+    float logit_new, log_ratio;
+    split(sigmoidf(L.logit[s]), multiplicity(L.counts, s, L.grow), logit_new, log_ratio);
+    R.logit[s] = logit_new;
+    for (int k = 0; k < R.scales_width; ++k) R.log_scales[s * R.scales_width + k] += log_ratio;
 }
 
 inline int64_t scan_blocks(int64_t n) { return ceil_div(n, kScanBlock); }
@@ -449,15 +505,16 @@ struct McmcWs {
     McmcTotals *tot;
     double *blk_w, *blk_o, *cdf;
     int64_t *blk_dead;
-    int32_t *blk_bad, *counts, *src;
+    int32_t *blk_bad, *counts, *dst;
+    uint32_t *src;
 };
 
-// src holds one source per row (relocate) or per draw (grow).
+// src and dst (relocate) hold one row per draw: at most n, or n_draw for grow.
 inline int64_t mcmc_ws_bytes(int64_t n, int64_t n_draw) {
     const int64_t nb = scan_blocks(n);
     return align256(sizeof(McmcTotals)) + 2 * align256(8 * nb) + align256(8 * nb) +
            align256(4 * nb) + align256(8 * n) + align256(4 * n) +
-           align256(4 * (n > n_draw ? n : n_draw));
+           2 * align256(4 * (n > n_draw ? n : n_draw));
 }
 
 inline McmcWs mcmc_ws(void *ws, int64_t n, int64_t n_draw) {
@@ -471,51 +528,61 @@ inline McmcWs mcmc_ws(void *ws, int64_t n, int64_t n_draw) {
     W.blk_bad = (int32_t *)p; p += align256(4 * nb);
     W.cdf = (double *)p; p += align256(8 * n);
     W.counts = (int32_t *)p; p += align256(4 * n);
-    W.src = (int32_t *)p;
+    W.src = (uint32_t *)p; p += align256(4 * (n > n_draw ? n : n_draw));
+    W.dst = (int32_t *)p;
     return W;
 }
 
-static int32_t row_tensors(RowTensors &R, int32_t n_tensors, float *const *tensors,
-                           const int32_t *widths, const int32_t *kinds, const char *who) {
+// The tasks over n list rows, the widest tensors' first.
+static int32_t row_tasks(RowTasks &R, int64_t n, int32_t n_tensors, float *const *tensors,
+                         const int32_t *widths, const int32_t *kinds, const char *who) {
     MG_REQUIRE(n_tensors >= 1 && n_tensors <= kMaxTensors, "%s: %d tensors (1..%d)", who,
                n_tensors, kMaxTensors);
     MG_REQUIRE(tensors && widths && kinds, "%s: null tensor table", who);
     int n_logit = 0, n_scales = 0;
+    int order[kMaxTensors];
     for (int t = 0; t < n_tensors; ++t) {
         MG_REQUIRE(tensors[t] != nullptr, "%s: tensor %d is null", who, t);
         MG_REQUIRE(widths[t] >= 1, "%s: tensor %d has row width %d", who, t, widths[t]);
         MG_REQUIRE(kinds[t] >= 0 && kinds[t] <= 3, "%s: tensor %d kind %d", who, t, kinds[t]);
         MG_REQUIRE(kinds[t] != 2 || widths[t] == 1, "%s: the logit tensor has width %d", who,
                    widths[t]);
-        R.p[t] = tensors[t];
-        R.width[t] = widths[t];
-        R.kind[t] = kinds[t];
-        n_logit += kinds[t] == 2;
-        n_scales += kinds[t] == 1;
+        if (kinds[t] == 1) {
+            R.log_scales = tensors[t];
+            R.scales_width = widths[t];
+            ++n_scales;
+        }
+        if (kinds[t] == 2) {
+            R.logit = tensors[t];
+            ++n_logit;
+        }
+        int k = t;
+        for (; k > 0 && widths[order[k - 1]] < widths[t]; --k) order[k] = order[k - 1];
+        order[k] = t;
     }
     MG_REQUIRE(n_logit == 1 && n_scales == 1,
                "%s: need exactly one logit-opacity and one log-scales tensor", who);
-    // Copied tensors first for the source update's concatenation: order the
-    // table so kinds 1-3 form a suffix, then give both column maps.
-    RowTensors S{};
-    int k = 0;
-    for (int pass = 0; pass < 2; ++pass)
-        for (int t = 0; t < n_tensors; ++t)
-            if ((R.kind[t] == 0) == (pass == 0)) {
-                S.p[k] = R.p[t]; S.width[k] = R.width[t]; S.kind[k] = R.kind[t]; ++k;
-            }
-    S.count = n_tensors;
-    int cols = 0, src_cols = 0;
-    for (int t = 0; t < n_tensors; ++t) {
-        S.col0[t] = cols;
-        cols += S.width[t];
-        // Copied tensors take no source columns: they map below column 0.
-        S.src_col0[t] = S.kind[t] == 0 ? -(1 << 30) : src_cols;
-        if (S.kind[t] != 0) src_cols += S.width[t];
+    int64_t blocks = 0;
+    auto add = [&](int t, int op) {
+        const int c = R.count++, w = widths[t];
+        R.p[c] = tensors[t];
+        R.width[c] = w;
+        R.op[c] = op;
+        R.rows[c] = w < kRowElems ? kRowElems / w : 1;
+        R.block0[c] = (uint32_t)blocks;
+        blocks += ceil_div(n, R.rows[c]);
+        R.block0[c + 1] = (uint32_t)blocks;
+    };
+    for (int k = 0; k < n_tensors; ++k) {
+        const int t = order[k];
+        if (kinds[t] == 3) {
+            add(t, kZeroSrc);
+            add(t, kZeroDst);
+        } else {
+            add(t, kinds[t] == 0 ? kCopy : kinds[t] == 1 ? kCopyScales : kCopyLogit);
+        }
     }
-    S.cols = cols;
-    S.src_cols = src_cols;
-    R = S;
+    MG_REQUIRE(blocks < (1LL << 31), "%s: %lld rows are too many", who, (long long)n);
     return MG_OK;
 }
 
@@ -589,8 +656,8 @@ int32_t mg_mcmc_apply(int64_t n, const float *logit_opac, const float *weights, 
                (long long)n_dest, (long long)n_draw);
     MG_REQUIRE(grow ? n_dest == n_draw : n_draw >= n,
                "mg_mcmc_apply: relocate needs a draw slot per row");
-    RowTensors R{};
-    int32_t rc = row_tensors(R, n_tensors, tensors, widths, kinds, "mg_mcmc_apply");
+    RowTasks R{};
+    int32_t rc = row_tasks(R, n_dest, n_tensors, tensors, widths, kinds, "mg_mcmc_apply");
     if (rc != MG_OK) return rc;
     McmcWs Wk = mcmc_ws(ws, n, n_draw);
     WeightArgs W{logit_opac, weights, n, thresh, grow, use_opacity};
@@ -598,33 +665,20 @@ int32_t mg_mcmc_apply(int64_t n, const float *logit_opac, const float *weights, 
     const int64_t nb = scan_blocks(n);
     TimedScope ts("mcmc_apply", s);
     mcmc_cdf_kernel<<<(unsigned)nb, kScanThreads, 0, s>>>(
-        W, use_opacity ? Wk.blk_o : Wk.blk_w, Wk.cdf);
+        W, use_opacity ? Wk.blk_o : Wk.blk_w, Wk.blk_dead, Wk.cdf, Wk.dst);
     MG_LAUNCHED("mcmc_cdf_kernel");
-    DrawArgs D{W, Wk.cdf, grow ? n_draw : 0, seed, 0x7069636bull /* stream tag */, Wk.src,
-               Wk.counts};
-    const int64_t n_cand = grow ? n_draw : n;
-    mcmc_draw_kernel<<<(unsigned)ceil_div(n_cand, 256), 256, 0, s>>>(D);
-    MG_LAUNCHED("mcmc_draw_kernel");
     if (n_dest > 0) {
-        // About one selected row per wave: copies are n_dest of n_cand
-        // candidates, sources at most n_dest of n rows.
-        auto chunk_for = [](int64_t sel, int64_t cand) {
-            int c = 4;
-            while (c < 256 && (double)c * (double)sel < 4.0 * (double)cand) c *= 2;
-            return c;
-        };
-        const int cc = chunk_for(n_dest, n_cand), cs = chunk_for(n_dest, n);
-        // Every copy reads its source before the sources are rewritten.
-        if (grow)
-            mcmc_rows_kernel<kGrowCopies><<<(unsigned)ceil_div(n_cand, cc), 256, 0, s>>>(
-                R, Wk.src, Wk.counts, logit_opac, n_cand, dst0, 1, cc);
-        else
-            mcmc_rows_kernel<kRelocateCopies><<<(unsigned)ceil_div(n_cand, cc), 256, 0, s>>>(
-                R, Wk.src, Wk.counts, logit_opac, n_cand, 0, 0, cc);
+        DrawArgs D{W, Wk.cdf, n_dest, seed, 0x7069636bull /* stream tag */, Wk.dst,
+                   grow ? nullptr : Wk.tot, Wk.src, Wk.counts};
+        mcmc_draw_kernel<<<(unsigned)ceil_div(n_dest, 256), 256, 0, s>>>(D);
+        MG_LAUNCHED("mcmc_draw_kernel");
+        const RowList L{grow ? nullptr : Wk.dst, Wk.src, Wk.counts, logit_opac, n_dest, dst0, grow,
+                        grow ? nullptr : Wk.tot};
+        mcmc_rows_kernel<<<R.block0[R.count], 256, 0, s>>>(R, L);
         MG_LAUNCHED("mcmc_rows_kernel");
-        mcmc_rows_kernel<kSources><<<(unsigned)ceil_div(n, cs), 256, 0, s>>>(
-            R, Wk.src, Wk.counts, logit_opac, n, 0, grow, cs);
-        MG_LAUNCHED("mcmc_rows_kernel");
+        // Every copy has read its source before the sources are rewritten.
+        mcmc_sources_kernel<<<(unsigned)ceil_div(n_dest, 256), 256, 0, s>>>(R, L);
+        MG_LAUNCHED("mcmc_sources_kernel");
     }
     return MG_OK;
 }

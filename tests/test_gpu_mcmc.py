@@ -289,3 +289,48 @@ def test_cpu_tensors_are_refused():
     p = make_params(10, 0.5)
     with pytest.raises(RuntimeError, match="ROCm"):
         mcmc.relocate(p)
+
+
+@pytest.mark.parametrize("mode", ["grow", "relocate"])
+@pytest.mark.parametrize("n", [3, 1025, 40_000])
+def test_rows_of_every_width_move_together(dev, n, mode):
+    """Copied tensors of widths around the kernel's run of 2048 elements: each
+    destination holds one live source's row in all of them, every other row is
+    as it was, and the state of destinations and sources is zero."""
+    from metal_gauss_amd import FusedAdam, mcmc
+
+    widths = (1, 3, 45, 2047, 2048, 2049) if n < 2000 else (1, 7, 45)
+    g = torch.Generator().manual_seed(n)
+    ids = torch.arange(n, dtype=torch.float32)
+    gp = {"logit_opac": torch.randn(n, generator=g).to(dev),
+          "log_scales": torch.randn(n, 3, generator=g).to(dev)}
+    gp.update({f"w{w}": ids[:, None].repeat(1, w).to(dev).requires_grad_(True) for w in widths})
+    opt = FusedAdam([gp[f"w{w}"] for w in widths])
+    for w in widths:
+        opt.state[gp[f"w{w}"]] = {"step": 1, "exp_avg": torch.ones(n, w, device=dev),
+                                  "exp_avg_sq": torch.ones(n, w, device=dev)}
+    if mode == "grow":
+        active = n - max(1, n // 3)
+        dst = torch.arange(active, n)
+        assert mcmc.grow(gp, target=n, active=active, opt=opt, seed=5) == n
+    else:
+        dst = torch.arange(0, n, 3)
+        gp["logit_opac"][dst.to(dev)] = -9.0
+        assert mcmc.relocate(gp, opt=opt, seed=5) == len(dst)
+    src = gp["w1"].detach()[dst.to(dev), 0].cpu().long()
+    live = torch.ones(n, dtype=torch.bool)
+    live[dst] = False
+    assert bool(live[src].all())
+    want = ids.clone()
+    want[dst] = src.float()
+    touched = ~live
+    touched[src] = True
+    for w in widths:
+        p = gp[f"w{w}"].detach().cpu()
+        assert torch.equal(p, want[:, None].expand(n, w)), w
+        for key in ("exp_avg", "exp_avg_sq"):
+            m = opt.state[gp[f"w{w}"]][key].cpu()
+            assert torch.equal(m, (~touched).float()[:, None].expand(n, w)), (w, key)
+    # A destination and its source share the split opacity.
+    logit = gp["logit_opac"].cpu()
+    assert torch.equal(logit[dst], logit[src])
