@@ -594,7 +594,7 @@ int32_t mg_ssim_chain_backward(const float *x, const float *y,
                                const float *d_stack, int32_t H, int32_t W,
                                float *d_x, mg_stream_t stream);
 
-/* Fused SSIM: one pass builds the five moments, blurs both ways in LDS and
+/* Fused SSIM: one pass builds the moments, blurs both ways in LDS and
  * evaluates SSIM; it writes the mean SSIM to mean_out (device, 1 float) and
  * the three unscaled adjoint maps (9,H,W) the backward needs to partials.
  * No counterpart in the reference, which runs the five kernels above

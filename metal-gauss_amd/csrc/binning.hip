@@ -1788,14 +1788,6 @@ struct TdShared {
     uint32_t red[2 * kTdWaves];
 };
 
-// Waits until this wave's outstanding LDS reads have returned. Needed before
-// a barrier after which other waves overwrite what this wave has read: the
-// barrier's own fence waits for LDS writes, not for reads whose values are
-// first used after it.
-__device__ __forceinline__ void lds_reads_done() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-}
-
 // Workgroup min and max of the keys.
 __device__ __forceinline__ void td_minmax(uint32_t &kmin, uint32_t &kmax, uint32_t *red) {
     for (int o = 32; o >= 1; o >>= 1) {

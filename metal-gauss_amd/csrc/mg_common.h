@@ -119,6 +119,14 @@ __device__ __forceinline__ int rank_in(uint64_t mask) {
                                      __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
 }
 
+// Waits until this wave's outstanding LDS reads have returned. Needed before
+// a barrier after which other waves overwrite what this wave has read: the
+// barrier's own fence waits for LDS writes, not for reads whose values are
+// first used after it.
+__device__ __forceinline__ void lds_reads_done() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+
 template <int CTRL, int ROW_MASK = 0xf>
 __device__ __forceinline__ float dpp_f(float v) {
     return __builtin_bit_cast(

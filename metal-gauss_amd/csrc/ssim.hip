@@ -5,7 +5,7 @@
 //   * the five kernels of the reference's ABI (metal_gauss/csrc/ssim.metal:
 //     23-188), same layouts: (H,W,3) images and (15,H,W) moment stacks;
 //   * a fused pair. The forward loads an image tile with a 5-pixel halo into
-//     LDS, forms the five moments, blurs them horizontally then vertically in
+//     LDS, forms the moments, blurs them horizontally then vertically in
 //     LDS, evaluates SSIM and writes the three adjoint maps the backward needs
 //     (per colour: dS/dmx, dS/dE[xx], dS/dE[xy], unscaled); the backward blurs
 //     those maps the same way (the window is symmetric, so the blur is its own
@@ -68,21 +68,6 @@ __global__ void ssim_blur15_kernel(const float *src, const float *w, int dir, in
     dst[base + (int64_t)py * W + px] = s;
 }
 
-__device__ __forceinline__ void ssim_terms(float mx, float my, float exx, float eyy, float exy,
-                                           float &S, float &p_mx, float &p_xx, float &p_xy) {
-    const float sxx = exx - mx * mx, syy = eyy - my * my, sxy = exy - mx * my;
-    const float A = 2.0f * mx * my + kSsimC1;
-    const float B = 2.0f * sxy + kSsimC2;
-    const float C = mx * mx + my * my + kSsimC1;
-    const float D = sxx + syy + kSsimC2;
-    const float invCD = 1.0f / (C * D);
-    S = A * B * invCD;
-    const float dA = B * invCD, dB = A * invCD, dC = -S / C, dD = -S / D;
-    p_xy = 2.0f * dB;
-    p_xx = dD;
-    p_mx = 2.0f * my * (dA - dB) + 2.0f * mx * (dC - dD);
-}
-
 __global__ void ssim_tail_fwd_kernel(const float *b, int64_t npix, float *out) {
     const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (gid >= 3 * npix) return;
@@ -129,22 +114,37 @@ __global__ void ssim_chain_bwd_kernel(const float *x, const float *y, const floa
 }
 
 // ------------------------------------------------------------- fused kernels
-constexpr int kTW = 32, kTH = 16;                 // output tile
-constexpr int kIW = kTW + 2 * kR, kIH = kTH + 2 * kR;   // 42 x 26 with halo
+// Vector issue bounds both kernels, so the split is chosen for the fewest
+// instructions a pixel. Tiles of 32x32 blur 42 rows horizontally for 32 rows
+// of output (tiles of 32x16 blurred 26 for 16); a horizontal task makes eight
+// outputs from 18 inputs and a vertical one four from 14; S needs E[xx] and
+// E[yy] only as their sum, so the forward blurs four maps and not five (the
+// sum as that of (x - y)^2 and 2 xy, see ssim_terms); its
+// three quotients share two reciprocals; and a thread's halo loads lie in one
+// column, so its index is formed once. The blurred maps overwrite their inputs
+// in LDS (21.5 instead of 36.3 KB: six workgroups a CU instead of four, 54 ->
+// 50 us for the forward at 1920x1080). Forward and backward: 63 + 46 -> 50 +
+// 34.5 us at 1920x1080, 24.5 + 18.5 -> 20.2 + 16.1 at 800x800.
+constexpr int kTW = 32, kTH = 32;                 // output tile
+constexpr int kIW = kTW + 2 * kR, kIH = kTH + 2 * kR;   // 42 x 42 with halo
 constexpr int kIWP = 44;                          // LDS row stride: 16-byte rows
 constexpr int kSsimThreads = 256;
 // Register blocking of the separable blur: a horizontal task makes kHRun
 // neighbouring outputs of one row from one read of its kHRun + 2 kR inputs;
 // a vertical task makes kVRun outputs of one column.
-constexpr int kHRun = 4, kVRun = 2;
-constexpr int kHTasks = kIH * (kTW / kHRun);      // 208
+constexpr int kHRun = 8, kVRun = 4;
+constexpr int kHIn = 20;                          // inputs read: five float4s
+constexpr int kHTasks = kIH * (kTW / kHRun);      // 168
 constexpr int kVTasks = (kTH / kVRun) * kTW;      // 256
 static_assert(kHTasks <= kSsimThreads && kVTasks == kSsimThreads, "blur tasks per thread");
-static_assert(kHRun + 2 * kR <= 16 && (kTW / kHRun - 1) * kHRun + 16 <= kIWP,
-              "a horizontal task reads four float4s of its row");
-// Halo elements per thread: all of a thread's loads are requested before any
-// of them is stored to LDS (a rolled loop waits for each in turn).
-constexpr int kLoadIters = (kIH * kIW + kSsimThreads - 1) / kSsimThreads;   // 5
+static_assert(kHRun + 2 * kR <= kHIn && (kTW / kHRun - 1) * kHRun + kHIn <= kIWP,
+              "a horizontal task reads five float4s of its row");
+// Halo elements per thread: thread t loads column t % kIW of rows t / kIW + 6 r
+// (252 of the 256 threads), all requested before any of them is stored to LDS
+// (a rolled loop waits for each in turn).
+constexpr int kLoadRows = kSsimThreads / kIW;     // 6
+constexpr int kLoadIters = kIH / kLoadRows;       // 7
+static_assert(kLoadRows * kLoadIters == kIH, "whole rows of loads");
 
 // Work items of the fused kernels: (output tile, channel) pairs, item =
 // 3 * tile + channel, tile = ty * tiles_x + tx. The items are dealt to the XCDs
@@ -161,14 +161,14 @@ __device__ __forceinline__ SsimItem ssim_item(int tiles_x) {
 }
 
 // The horizontal task of thread t: row t / (kTW / kHRun), first output column
-// kHRun * (t % (kTW / kHRun)); its inputs are 16 floats of that LDS row from
+// kHRun * (t % (kTW / kHRun)); its inputs are kHIn floats of that LDS row from
 // the same column.
 __device__ __forceinline__ void h_inputs(const float (*src)[kIWP], int t, int &row, int &c0,
-                                         float (&v)[16]) {
+                                         float (&v)[kHIn]) {
     row = t / (kTW / kHRun);
     c0 = kHRun * (t % (kTW / kHRun));
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < kHIn / 4; ++q) {
         const float4 f = *reinterpret_cast<const float4 *>(&src[row][c0 + 4 * q]);
         v[4 * q] = f.x;
         v[4 * q + 1] = f.y;
@@ -177,14 +177,43 @@ __device__ __forceinline__ void h_inputs(const float (*src)[kIWP], int t, int &r
     }
 }
 
+// The SSIM of a pixel and its adjoints from the blurred x, y, (x - y)^2 and xy.
+// sxx + syy is the variance of x - y plus 2 sxy: where the images are alike
+// the variance is small and the rounding of sxy, a difference of blurred
+// products, enters numerator and denominator alike.
+__device__ __forceinline__ void ssim_terms(float mx, float my, float edd, float exy, float &S,
+                                           float &p_mx, float &p_xx, float &p_xy) {
+    const float mxy = mx * my, dm = mx - my;
+    const float A = 2.0f * mxy + kSsimC1;
+    const float B = 2.0f * (exy - mxy) + kSsimC2;
+    const float C = mx * mx + my * my + kSsimC1;
+    const float D = (edd - dm * dm) + B;
+    const float iC = 1.0f / C, iD = 1.0f / D;
+    const float dA = B * iC * iD, dB = A * iC * iD;
+    S = A * dA;
+    const float dC = -S * iC, dD = -S * iD;
+    p_xy = 2.0f * dB;
+    p_xx = dD;
+    p_mx = 2.0f * my * (dA - dB) + 2.0f * mx * (dC - dD);
+}
+
 // block_sums[b] gets work item b's SSIM sum; with l1_sums, l1_sums[b] gets
 // its sum of |x - y| over the same pixels and channel.
-__global__ __launch_bounds__(kSsimThreads) void ssim_fused_fwd_kernel(
+__global__ __launch_bounds__(kSsimThreads) __attribute__((amdgpu_waves_per_eu(6))) void
+ssim_fused_fwd_kernel(
     const float *x, const float *y, const float *__restrict__ w, int H, int W, int tiles_x,
     float *partials, float *block_sums, float *l1_sums) {
-    __shared__ __align__(16) float s_x[kIH][kIWP];
-    __shared__ __align__(16) float s_y[kIH][kIWP];
-    __shared__ __align__(16) float s_h[5][kIH][kTW];
+    // The horizontal pass's maps take the images' place: every task holds its
+    // results in registers across a barrier.
+    __shared__ __align__(16) union {
+        struct {
+            float x[kIH][kIWP], y[kIH][kIWP];
+        } in;
+        float h[4][kIH][kTW];
+    } u;
+    float(*const s_x)[kIWP] = u.in.x;
+    float(*const s_y)[kIWP] = u.in.y;
+    float(*const s_h)[kIH][kTW] = u.h;
     __shared__ float s_red[2][kSsimThreads / 64];
     const SsimItem it = ssim_item(tiles_x);
     const int c = it.c;
@@ -195,26 +224,24 @@ __global__ __launch_bounds__(kSsimThreads) void ssim_fused_fwd_kernel(
     for (int k = 0; k <= 2 * kR; ++k) wk[k] = w[k];
     {
         float xv[kLoadIters], yv[kLoadIters];
+        const int ly = tid / kIW, lx = tid - ly * kIW, gx = x0 + lx;
+        const bool col = ly < kLoadRows && gx >= 0 && gx < W;
 #pragma unroll
         for (int r = 0; r < kLoadIters; ++r) {
-            const int i = tid + r * kSsimThreads;
-            const int ly = i / kIW, lx = i - ly * kIW;
-            const int gx = x0 + lx, gy = y0 + ly;
+            const int gy = y0 + ly + kLoadRows * r;
             xv[r] = 0.f;
             yv[r] = 0.f;
-            if (i < kIH * kIW && gx >= 0 && gx < W && gy >= 0 && gy < H) {
+            if (col && gy >= 0 && gy < H) {
                 const int64_t o = ((int64_t)gy * W + gx) * 3 + c;
                 xv[r] = x[o];
                 yv[r] = y[o];
             }
         }
+        if (ly < kLoadRows) {
 #pragma unroll
-        for (int r = 0; r < kLoadIters; ++r) {
-            const int i = tid + r * kSsimThreads;
-            if (i < kIH * kIW) {
-                const int ly = i / kIW, lx = i - ly * kIW;
-                s_x[ly][lx] = xv[r];
-                s_y[ly][lx] = yv[r];
+            for (int r = 0; r < kLoadIters; ++r) {
+                s_x[ly + kLoadRows * r][lx] = xv[r];
+                s_y[ly + kLoadRows * r][lx] = yv[r];
             }
         }
     }
@@ -226,62 +253,71 @@ __global__ __launch_bounds__(kSsimThreads) void ssim_fused_fwd_kernel(
         s_y[ly][lx] = 0.f;
     }
     __syncthreads();
-    // Horizontal pass over the full halo height: each input's x, y, x^2,
-    // y^2 and xy once, into the kHRun outputs whose window holds it.
+    // Horizontal pass over the full halo height: each input's x, y, (x - y)^2
+    // and xy once, into the kHRun outputs whose window holds it.
+    float local = 0.f, local_l1 = 0.f;
+    const int lx = tid % kTW, r0 = kVRun * (tid / kTW);
+    const int gx = it.tx * kTW + lx;
+#pragma unroll
+    for (int o = 0; o < kVRun; ++o) {
+        const float l1 = fabsf(s_x[r0 + o + kR][lx + kR] - s_y[r0 + o + kR][lx + kR]);
+        local_l1 += gx < W && it.ty * kTH + r0 + o < H ? l1 : 0.f;
+    }
+    int row = 0, c0 = 0;
+    float m[4][kHRun] = {};
     if (tid < kHTasks) {
-        int row, c0;
-        float xv[16], yv[16];
+        float xv[kHIn], yv[kHIn];
         h_inputs(s_x, tid, row, c0, xv);
         h_inputs(s_y, tid, row, c0, yv);
-        float m[5][kHRun] = {};
 #pragma unroll
         for (int j = 0; j < kHRun + 2 * kR; ++j) {
-            const float a = xv[j], b = yv[j], aa = a * a, bb = b * b, ab = a * b;
+            const float a = xv[j], b = yv[j], dd = (a - b) * (a - b), ab = a * b;
 #pragma unroll
             for (int o = 0; o < kHRun; ++o) {
                 const int k = j - o;
                 if (k < 0 || k > 2 * kR) continue;
                 m[0][o] = fmaf(wk[k], a, m[0][o]);
                 m[1][o] = fmaf(wk[k], b, m[1][o]);
-                m[2][o] = fmaf(wk[k], aa, m[2][o]);
-                m[3][o] = fmaf(wk[k], bb, m[3][o]);
-                m[4][o] = fmaf(wk[k], ab, m[4][o]);
+                m[2][o] = fmaf(wk[k], dd, m[2][o]);
+                m[3][o] = fmaf(wk[k], ab, m[3][o]);
             }
         }
+    }
+    lds_reads_done();
+    __syncthreads();
+    if (tid < kHTasks) {
 #pragma unroll
-        for (int q = 0; q < 5; ++q)
-            *reinterpret_cast<float4 *>(&s_h[q][row][c0]) =
-                make_float4(m[q][0], m[q][1], m[q][2], m[q][3]);
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int h = 0; h < kHRun; h += 4)
+                *reinterpret_cast<float4 *>(&s_h[q][row][c0 + h]) =
+                    make_float4(m[q][h], m[q][h + 1], m[q][h + 2], m[q][h + 3]);
     }
     __syncthreads();
     // Vertical pass and the SSIM tail: thread t makes rows kVRun * (t / kTW)
     // + [0, kVRun) of column t % kTW.
     const int64_t N = (int64_t)W * H;
-    float local = 0.f, local_l1 = 0.f;
     {
-        const int lx = tid % kTW, r0 = kVRun * (tid / kTW);
-        float m[kVRun][5] = {};
+        float m[kVRun][4] = {};
 #pragma unroll
         for (int j = 0; j < kVRun + 2 * kR; ++j) {
-            float h[5];
+            float h[4];
 #pragma unroll
-            for (int q = 0; q < 5; ++q) h[q] = s_h[q][r0 + j][lx];
+            for (int q = 0; q < 4; ++q) h[q] = s_h[q][r0 + j][lx];
 #pragma unroll
             for (int o = 0; o < kVRun; ++o) {
                 const int k = j - o;
                 if (k < 0 || k > 2 * kR) continue;
 #pragma unroll
-                for (int q = 0; q < 5; ++q) m[o][q] = fmaf(wk[k], h[q], m[o][q]);
+                for (int q = 0; q < 4; ++q) m[o][q] = fmaf(wk[k], h[q], m[o][q]);
             }
         }
-        const int gx = it.tx * kTW + lx;
 #pragma unroll
         for (int o = 0; o < kVRun; ++o) {
-            const int ly = r0 + o, gy = it.ty * kTH + ly;
+            const int gy = it.ty * kTH + r0 + o;
             if (gx >= W || gy >= H) continue;
-            local_l1 += fabsf(s_x[ly + kR][lx + kR] - s_y[ly + kR][lx + kR]);
             float S, pm, pxx, pxy;
-            ssim_terms(m[o][0], m[o][1], m[o][2], m[o][3], m[o][4], S, pm, pxx, pxy);
+            ssim_terms(m[o][0], m[o][1], m[o][2], m[o][3], S, pm, pxx, pxy);
             local += S;
             const int64_t po = (int64_t)gy * W + gx;
             partials[(0 + c) * N + po] = pm;
@@ -383,11 +419,17 @@ __global__ __launch_bounds__(256) void photometric_loss_kernel(const float *ssim
 // dx = g / (3N) * (a_ssim * dSSIM_sum/dx + a_l1 * sign(x - y)), g = scale_dev[0]:
 // a_ssim = 1, a_l1 = 0 is the gradient of the SSIM mean; a_ssim = -lam,
 // a_l1 = 1 - lam that of the photometric loss.
-__global__ __launch_bounds__(kSsimThreads) void ssim_fused_bwd_kernel(
+__global__ __launch_bounds__(kSsimThreads) __attribute__((amdgpu_waves_per_eu(6))) void
+ssim_fused_bwd_kernel(
     const float *x, const float *y, const float *__restrict__ w, const float *partials,
     const float *scale_dev, int H, int W, int tiles_x, float a_ssim, float a_l1, float *dx) {
-    __shared__ __align__(16) float s_p[3][kIH][kIWP];
-    __shared__ __align__(16) float s_h[3][kIH][kTW];
+    // As in the forward, the blurred maps take their inputs' place.
+    __shared__ __align__(16) union {
+        float p[3][kIH][kIWP];
+        float h[3][kIH][kTW];
+    } u;
+    float(*const s_p)[kIH][kIWP] = u.p;
+    float(*const s_h)[kIH][kTW] = u.h;
     const SsimItem it = ssim_item(tiles_x);
     const int c = it.c;
     const int x0 = it.tx * kTW - kR, y0 = it.ty * kTH - kR;
@@ -398,27 +440,24 @@ __global__ __launch_bounds__(kSsimThreads) void ssim_fused_bwd_kernel(
     for (int k = 0; k <= 2 * kR; ++k) wk[k] = w[k];
     {
         float pv[3][kLoadIters];
+        const int ly = tid / kIW, lx = tid - ly * kIW, gx = x0 + lx;
+        const bool col = ly < kLoadRows && gx >= 0 && gx < W;
 #pragma unroll
         for (int r = 0; r < kLoadIters; ++r) {
-            const int i = tid + r * kSsimThreads;
-            const int ly = i / kIW, lx = i - ly * kIW;
-            const int gx = x0 + lx, gy = y0 + ly;
+            const int gy = y0 + ly + kLoadRows * r;
 #pragma unroll
             for (int q = 0; q < 3; ++q) pv[q][r] = 0.f;
-            if (i < kIH * kIW && gx >= 0 && gx < W && gy >= 0 && gy < H) {
+            if (col && gy >= 0 && gy < H) {
                 const int64_t o = (int64_t)gy * W + gx;
 #pragma unroll
                 for (int q = 0; q < 3; ++q) pv[q][r] = partials[(3 * q + c) * N + o];
             }
         }
+        if (ly < kLoadRows) {
 #pragma unroll
-        for (int r = 0; r < kLoadIters; ++r) {
-            const int i = tid + r * kSsimThreads;
-            if (i < kIH * kIW) {
-                const int ly = i / kIW, lx = i - ly * kIW;
+            for (int r = 0; r < kLoadIters; ++r)
 #pragma unroll
-                for (int q = 0; q < 3; ++q) s_p[q][ly][lx] = pv[q][r];
-            }
+                for (int q = 0; q < 3; ++q) s_p[q][ly + kLoadRows * r][lx] = pv[q][r];
         }
     }
     for (int i = tid; i < kIH * (kIWP - kIW); i += kSsimThreads) {
@@ -428,12 +467,12 @@ __global__ __launch_bounds__(kSsimThreads) void ssim_fused_bwd_kernel(
         s_p[2][ly][lx] = 0.f;
     }
     __syncthreads();
+    int row = 0, c0 = 0;
+    float hm[3][kHRun] = {};
     if (tid < kHTasks) {
-        int row, c0;
-        float v[3][16];
+        float v[3][kHIn];
 #pragma unroll
         for (int q = 0; q < 3; ++q) h_inputs(s_p[q], tid, row, c0, v[q]);
-        float m[3][kHRun] = {};
 #pragma unroll
         for (int j = 0; j < kHRun + 2 * kR; ++j) {
 #pragma unroll
@@ -441,13 +480,19 @@ __global__ __launch_bounds__(kSsimThreads) void ssim_fused_bwd_kernel(
                 const int k = j - o;
                 if (k < 0 || k > 2 * kR) continue;
 #pragma unroll
-                for (int q = 0; q < 3; ++q) m[q][o] = fmaf(wk[k], v[q][j], m[q][o]);
+                for (int q = 0; q < 3; ++q) hm[q][o] = fmaf(wk[k], v[q][j], hm[q][o]);
             }
         }
+    }
+    lds_reads_done();
+    __syncthreads();
+    if (tid < kHTasks) {
 #pragma unroll
         for (int q = 0; q < 3; ++q)
-            *reinterpret_cast<float4 *>(&s_h[q][row][c0]) =
-                make_float4(m[q][0], m[q][1], m[q][2], m[q][3]);
+#pragma unroll
+            for (int h = 0; h < kHRun; h += 4)
+                *reinterpret_cast<float4 *>(&s_h[q][row][c0 + h]) =
+                    make_float4(hm[q][h], hm[q][h + 1], hm[q][h + 2], hm[q][h + 3]);
     }
     __syncthreads();
     const float scale = scale_dev[0] / (float)(3 * N);
@@ -487,6 +532,13 @@ __global__ __launch_bounds__(kSsimThreads) void ssim_fused_bwd_kernel(
 inline int64_t ssim_blocks(int H, int W) {
     return ceil_div(W, kTW) * ceil_div(H, kTH) * 3;
 }
+
+// The block sums a caller's workspace and the static scratch are sized by: one
+// per 32x16 pixels and channel, of which the 32x32 tiles use half.
+inline int64_t ssim_sized_blocks(int H, int W) {
+    return ceil_div(W, 32) * ceil_div(H, 16) * 3;
+}
+static_assert(kTW >= 32 && kTH >= 16, "no more tiles than sized");
 
 // ------------------------------------------------ allocation-free variant
 // mg_photometric_loss_forward_noalloc keeps the loss forward's block sums in
@@ -609,7 +661,7 @@ int32_t mg_ssim_chain_backward(const float *x, const float *y, const float *d_st
 
 int64_t mg_ssim_fused_workspace_bytes(int32_t H, int32_t W) {
     if (H <= 0 || W <= 0) return 0;
-    return 2 * ssim_blocks(H, W) * (int64_t)sizeof(float);   // SSIM and L1 block sums
+    return 2 * ssim_sized_blocks(H, W) * (int64_t)sizeof(float);   // SSIM and L1 block sums
 }
 
 int32_t mg_ssim_fused_forward(const float *x, const float *y, const float *w, int32_t H, int32_t W,
@@ -667,10 +719,11 @@ int32_t mg_photometric_loss_forward_noalloc(const float *x, const float *y, cons
                                             float *partials, float *out, mg_stream_t stream) {
     const char *who = "mg_photometric_loss_forward_noalloc";
     MG_REQUIRE(H > 0 && W > 0 && x && y && w && partials && out, "%s: bad arguments", who);
-    MG_REQUIRE(ssim_blocks(H, W) <= kStaticLossBlocks,
+    const int64_t tiles = ssim_sized_blocks(H, W);
+    MG_REQUIRE(tiles <= kStaticLossBlocks,
                "%s: a %dx%d image needs %lld block sums (3 per 32x16-pixel tile), more "
                "than the %lld the static scratch holds",
-               who, H, W, (long long)ssim_blocks(H, W), (long long)kStaticLossBlocks);
+               who, H, W, (long long)tiles, (long long)kStaticLossBlocks);
     float *sums = nullptr;
     const int32_t rc = static_scratch(&sums, who);
     if (rc != MG_OK) return rc;

@@ -115,3 +115,10 @@ def test_photometric_loss_upstream_gradient(dev):
     g1, = torch.autograd.grad(photometric_loss(a, b, w)[0], a)
     g2, = torch.autograd.grad(2.5 * photometric_loss(a, b, w)[0], a)
     assert torch.allclose(g2, 2.5 * g1, rtol=1e-5, atol=1e-12)
+
+
+@pytest.mark.parametrize("H,W", [(1, 1), (1, 64), (31, 33), (32, 32), (33, 31), (42, 43), (65, 5)])
+def test_photometric_loss_at_the_edges_of_tiles(dev, H, W):
+    """The same expression where an image ends inside, at and just past the
+    kernels' 32x32 tiles and their halo; bars as above."""
+    test_photometric_loss_matches_the_trainer_expression(dev, H, W, 0.2)
