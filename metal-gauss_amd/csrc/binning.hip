@@ -166,22 +166,65 @@ __device__ __forceinline__ int rec_walk(const BinRec &r, bool test, int tile, in
     return n;
 }
 
+// Quotients by one Gaussian's a and c: the correctly rounded reciprocals and
+// what rounding them lost.
+struct ClaimDiv {
+    float ia, ia_lo, ic, ic_lo;
+};
+
+// x / d, correctly rounded, from y = RN(1 / d) and y_lo = 1 / d - y: the first
+// quotient carries the reciprocal to twice the precision, so it is a faithful
+// rounding of x / d; the residual r of a faithful quotient is exact in an fma,
+// and q + r y rounds to RN(x / d) (Markstein's theorem). Four operations
+// instead of the general division's eleven and its reciprocal. It needs every
+// step free of over- and underflow: see quotients_safe.
+__device__ __forceinline__ float div_known(float x, float d, float y, float y_lo) {
+    const float q = __builtin_fmaf(x, y, x * y_lo);
+    const float r = __builtin_fmaf(-d, q, x);
+    return __builtin_fmaf(r, y, q);
+}
+
+// True when div_known gives the IEEE quotient of every b * (edge - centre) by
+// a and c: the diagonal in [2^-40, 2^20], |b| zero or in [2^-50, 2^20], the
+// centre's coordinates zero or in [2^-20, 2^20]. Edges are whole numbers below
+// 2^31, so a difference is zero or at least 2^-43 (an ulp of the centre), a
+// product zero or in [2^-93, 2^52], a quotient normal, and a residual a
+// multiple of 2^-139, above the smallest denormal. A zero quotient may lose
+// its sign, which no comparison below sees. False for NaN and infinities.
+__device__ __forceinline__ bool quotients_safe(const BinRec &r) {
+    const float b = fabsf(r.b), x = fabsf(r.ux), y = fabsf(r.uy);
+    return r.a >= 0x1p-40f && r.a <= 0x1p20f && r.c >= 0x1p-40f && r.c <= 0x1p20f &&
+           b <= 0x1p20f && (b >= 0x1p-50f || b == 0.0f) && x <= 0x1p20f &&
+           (x >= 0x1p-20f || x == 0.0f) && y <= 0x1p20f && (y >= 0x1p-20f || y == 0.0f);
+}
+
+__device__ __forceinline__ ClaimDiv claim_div(const BinRec &r) {
+#pragma clang fp contract(off)
+    ClaimDiv q;
+    q.ia = 1.0f / r.a;
+    q.ia_lo = __builtin_fmaf(-r.a, q.ia, 1.0f) * q.ia;
+    q.ic = 1.0f / r.c;
+    q.ic_lo = __builtin_fmaf(-r.c, q.ic, 1.0f) * q.ic;
+    return q;
+}
+
 // One tile's decision, with exactly the expressions rec_walk evaluates for it
 // (its shared edge minimisers are the same expressions of the same edge
 // lines), so a wave that splits a rectangle over its lanes decides every
-// tile as the walk does, bit for bit.
-__device__ __forceinline__ bool tile_claim(const BinRec &r, bool test, int tx, int ty, int tile,
-                                           int W, int H) {
+// tile as the walk does, bit for bit. div_a and div_c give the quotients by a
+// and c.
+template <typename DivA, typename DivC>
+__device__ __forceinline__ bool tile_claim_div(const BinRec &r, int tx, int ty, int tile, int W,
+                                               int H, DivA &&div_a, DivC &&div_c) {
 #pragma clang fp contract(off)
-    if (!test) return true;
     const float mux = r.ux, muy = r.uy, a = r.a, b = r.b, c = r.c;
     const float ry0 = (float)(ty * tile), ry1 = fminf((float)((ty + 1) * tile), (float)H);
     const float rx0 = (float)(tx * tile), rx1 = fminf((float)((tx + 1) * tile), (float)W);
     if (muy >= ry0 && muy <= ry1 && mux >= rx0 && mux <= rx1) return true;
-    const float u0 = mux - b * (ry0 - muy) / a;
-    const float u1 = mux - b * (ry1 - muy) / a;
-    const float v0 = muy - b * (rx0 - mux) / c;
-    const float v1 = muy - b * (rx1 - mux) / c;
+    const float u0 = mux - div_a(b * (ry0 - muy));
+    const float u1 = mux - div_a(b * (ry1 - muy));
+    const float v0 = muy - div_c(b * (rx0 - mux));
+    const float v1 = muy - div_c(b * (rx1 - mux));
     const float ey0 = ry0 - muy, ey1 = ry1 - muy;
     float ex = fminf(fmaxf(u0, rx0), rx1) - mux;
     float best = a * ex * ex + 2.0f * b * ex * ey0 + c * ey0 * ey0;
@@ -194,6 +237,14 @@ __device__ __forceinline__ bool tile_claim(const BinRec &r, bool test, int tx, i
     ex = rx1 - mux;
     best = fminf(best, a * ex * ex + 2.0f * b * ex * ey + c * ey * ey);
     return best < r.thr;
+}
+
+__device__ __forceinline__ bool tile_claim(const BinRec &r, bool test, int tx, int ty, int tile,
+                                           int W, int H) {
+    if (!test) return true;
+    return tile_claim_div(
+        r, tx, ty, tile, W, H, [&](float x) { return x / r.a; },
+        [&](float x) { return x / r.c; });
 }
 
 // Rectangles larger than this many tiles are walked by a whole wave instead
@@ -241,22 +292,35 @@ __device__ __forceinline__ uint32_t dpp_min_u32(uint32_t v) {
                                                         ROW_MASK, 0xf, false));
 }
 
+// floor(n / d) and ceil(n / d) of small whole numbers, 0 <= n (+ d) < 2^21 and
+// d >= 1: (n + 1/2) / d lies at least 1 / (2 d) from a whole number, and the
+// product with the 1-ulp reciprocal is off by less than 3 2^-24 (n + 1/2) / d.
+__device__ __forceinline__ int small_div(int n, int d) {
+    return (int)(((float)n + 0.5f) * __builtin_amdgcn_rcpf((float)d));
+}
+__device__ __forceinline__ int small_ceil_div(int n, int d) { return small_div(n + d - 1, d); }
+
+// Columns of a strip R rows high of a rectangle w wide.
+__device__ __forceinline__ int strip_cols(int w, int R) { return min(w, small_div(64, R)); }
+
+// A wave prices a rectangle in about 50 instructions; with IEEE divisions for
+// these quotients it was 130, a third of a rectangle of up to 64 tiles. The
+// write pass reads R from the kept mask instead (76M tiles in 1.33M
+// rectangles: the count pass 343 -> 290 us, the write pass 278 -> 227).
 __device__ __forceinline__ StripPlan strip_plan(const BinRec &r, int lane) {
     const int w = (int)(r.xs >> 16) - (int)(r.xs & 0xffffu) + 1;
     const int h = (int)(r.ys >> 16) - (int)(r.ys & 0xffffu) + 1;
     // Lane l prices R = l + 1 rows a step (strips of min(w, 64 / R)
     // columns); the wave takes the fewest steps, the smallest R on ties.
-    // The quotients of these small integers (w, h < 2^16, R <= 64) come from
-    // correctly rounded float divisions, exact after floor / ceil; the step
-    // count is held below 2^26 (beyond it any choice is as good), so the key
-    // steps << 6 | lane fits 32 bits and the minimum takes DPP row shifts
-    // and broadcasts rather than lane shuffles.
+    // The step count is held below 2^26 (beyond it any choice is as good), so
+    // the key steps << 6 | lane fits 32 bits and the minimum takes DPP row
+    // shifts and broadcasts rather than lane shuffles.
     uint32_t key;
     {
         const int R = lane + 1;
-        const int s = min(w, (int)(64.0f / (float)R));
-        const uint32_t ns = (uint32_t)ceilf((float)w / (float)s);
-        const uint32_t nr = (uint32_t)ceilf((float)h / (float)R);
+        const int s = strip_cols(w, R);
+        const uint32_t ns = (uint32_t)small_ceil_div(w, s);
+        const uint32_t nr = (uint32_t)small_ceil_div(h, R);
         const uint32_t steps = min(ns * nr, (1u << 26) - 1u);
         key = steps << 6 | (uint32_t)lane;
         key = dpp_min_u32<0x111>(key);        // row_shr:1
@@ -268,10 +332,10 @@ __device__ __forceinline__ StripPlan strip_plan(const BinRec &r, int lane) {
     }
     StripPlan P;
     P.R = (int)(__builtin_amdgcn_readlane(key, 63) & 63u) + 1;
-    P.s = min(w, (int)(64.0f / (float)P.R));
-    P.ns = (int)ceilf((float)w / (float)P.s);
-    P.nr = (int)ceilf((float)h / (float)P.R);
-    P.rg = (int)((float)lane / (float)P.s);
+    P.s = strip_cols(w, P.R);
+    P.ns = __builtin_amdgcn_readfirstlane(small_ceil_div(w, P.s));
+    P.nr = __builtin_amdgcn_readfirstlane(small_ceil_div(h, P.R));
+    P.rg = small_div(lane, P.s);
     P.cl = lane - P.rg * P.s;
     P.lane_ok = lane < P.R * P.s;
     return P;
@@ -355,19 +419,25 @@ __device__ __forceinline__ void strip_walk(const BinRec &r, const StripPlan &P, 
 // replays the steps instead of testing every tile again. A count workgroup
 // has kBlockWords words, taken by its rectangles as their walks start; a
 // rectangle whose steps no longer fit is walked again by the write pass.
-// Its mask word records where its words are: 1 + the first word's index,
-// plus the step count from bit kWordSteps (0: not kept).
+// Its mask word records where its words are: 1 + the first word's index, the
+// step count from bit kWordSteps and the walk's rows a step, less one, from
+// bit kWordRows (0: not kept).
 constexpr int kBlockWords = 1024;
-constexpr int kWordSteps = 11;
+constexpr int kWordSteps = 11, kWordRows = 22;
 static_assert(kBlockWords < (1 << kWordSteps), "the first word's index + 1 fits below the steps");
+static_assert(kBlockWords < (1 << (kWordRows - kWordSteps)), "the steps fit below the rows");
 
-__device__ __forceinline__ uint32_t kept_mask(int first, int nst) {
-    return (uint32_t)(first + 1) | ((uint32_t)nst << kWordSteps);
+__device__ __forceinline__ uint32_t kept_mask(int first, int nst, int R) {
+    return (uint32_t)(first + 1) | ((uint32_t)nst << kWordSteps) |
+           ((uint32_t)(R - 1) << kWordRows);
 }
 __device__ __forceinline__ int kept_first(uint32_t m) {
     return (int)(m & ((1u << kWordSteps) - 1u)) - 1;
 }
-__device__ __forceinline__ int kept_steps(uint32_t m) { return (int)(m >> kWordSteps); }
+__device__ __forceinline__ int kept_steps(uint32_t m) {
+    return (int)(m >> kWordSteps & ((1u << (kWordRows - kWordSteps)) - 1u));
+}
+__device__ __forceinline__ int kept_rows(uint32_t m) { return (int)(m >> kWordRows) + 1; }
 
 __device__ __forceinline__ int rec_area(const BinRec &r) {
     return ((int)(r.xs >> 16) - (int)(r.xs & 0xffffu) + 1) *
@@ -578,74 +648,106 @@ __device__ __forceinline__ int wave_incl_max(int v) {
     return v;
 }
 
+// Inclusive sum over the wave, in lane order, likewise.
+__device__ __forceinline__ int wave_incl_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);   // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);   // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);   // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31
+    return v;
+}
+
 // The small rectangles' tile tests of one wave, one (Gaussian, tile)
 // candidate per lane: a per-lane walk made every lane wait for the wave's
-// largest rectangle. Lane l's rectangle has ar tiles (0 for none) and its
-// candidates are [pre, pre + ar) of the wave's row; a candidate finds its
-// rectangle as the last head mark at or before it (an inclusive max over the
-// lanes), and its tile from its row-major index. Each tile's decision is
-// tile_claim, the walk's own expressions, so the result is bit for bit the
-// walk's. Returns this lane's claim mask (bit loc for tile loc).
+// largest rectangle. Lane l's rectangle has ar tiles (0 for none); the
+// rectangles that have any lie in lane order in the wave's slices, one's
+// candidates are [pre, pre + ar) of the wave's row with a mark at the first,
+// and a candidate's rectangle is the number of marks up to it. What a
+// candidate would divide by is a property of its rectangle and formed once
+// for it: the reciprocals of a and c (ClaimDiv) and of the width. The test is
+// arithmetic-bound, and dividing per candidate took about a third of it
+// (4.3M candidates, with strip_plan's divisions: the count pass 41 -> 32 us).
+// Each tile's decision is tile_claim's, the walk's own expressions, so the
+// result is bit for bit the walk's. Returns this lane's claim mask (bit loc
+// for tile loc).
+constexpr int kPreBits = 11, kFastBit = 28;
+static_assert(63 * kWaveWalkArea < (1 << kPreBits), "pre fits below the width's reciprocal");
+
 __device__ __forceinline__ uint32_t wave_small_claims(const BinRec &r, int ar, bool test,
                                                       int tile, int W, int H, BinRec *w_rec,
-                                                      int32_t *w_pre, uint32_t *w_msk,
-                                                      uint8_t *w_own, int lane) {
+                                                      float4 *w_div, uint32_t *w_pre,
+                                                      uint32_t *w_msk, uint8_t *w_own,
+                                                      int lane) {
     if (!test) return ar >= 32 ? 0xFFFFFFFFu : (1u << ar) - 1u;
-    int incl = ar;
-    for (int o = 1; o < 64; o <<= 1) {
-        const int t = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += t;
-    }
+    const int incl = wave_incl_sum(ar);
     const int pre = incl - ar;
-    const int total = __shfl(incl, 63, 64);
+    const int total = __builtin_amdgcn_readlane(incl, 63);
     if (total == 0) return 0u;   // wave-uniform
-    w_rec[lane] = r;
-    w_pre[lane] = pre;
-    w_msk[lane] = 0u;
+    const int rk = rank_in(ballot(ar > 0));
+    if (ar > 0) {
+        // loc < 32 and w <= 32: loc * ceil(2^16 / w) >> 16 is loc / w exactly.
+        const int w = (int)(r.xs >> 16) - (int)(r.xs & 0xffffu) + 1;
+        const uint32_t inv = (uint32_t)small_ceil_div(65536, w);
+        const ClaimDiv d = claim_div(r);
+        w_rec[rk] = r;
+        w_div[rk] = make_float4(d.ia, d.ia_lo, d.ic, d.ic_lo);
+        w_pre[rk] = (uint32_t)pre | inv << kPreBits |
+                    (quotients_safe(r) ? 1u << kFastBit : 0u);
+        w_msk[rk] = 0u;
+    }
     for (int i = lane; i < (total + 3) / 4; i += 64) reinterpret_cast<uint32_t *>(w_own)[i] = 0u;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (ar > 0) w_own[pre] = (uint8_t)(lane + 1);
+    if (ar > 0) w_own[pre] = (uint8_t)1;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    int carry = 0;
+    int before = -1;   // the last rectangle begun before this round
     for (int c0 = 0; c0 < total; c0 += 64) {
         const int c = c0 + lane;
         const bool valid = c < total;
-        const int h = valid ? (int)w_own[c] : 0;
-        const int own = max(wave_incl_max(h), carry);   // owner lane + 1 (>= 1 when valid)
-        carry = __shfl(own, 63, 64);
-        const int ol = max(own - 1, 0);
-        const BinRec q = w_rec[ol];
-        const int loc = c - w_pre[ol];
+        const bool head = valid && w_own[c] != 0;
+        const uint64_t hm = ballot(head);
+        // The first candidate is a head, so own >= 0.
+        const int own = before + rank_in(hm) + (head ? 1 : 0);
+        before += __popcll(hm);
+        const BinRec q = w_rec[own];
+        const float4 d = w_div[own];
+        const uint32_t pw = w_pre[own];
+        const int loc = c - (int)(pw & ((1u << kPreBits) - 1u));
         bool claim = false;
         if (valid) {
-            const int x0 = (int)(q.xs & 0xffffu), y0 = (int)(q.ys & 0xffffu);
-            const int w = (int)(q.xs >> 16) - x0 + 1;
-            // loc < 32 and w <= 32: loc * ceil(2^16 / w) >> 16 is loc / w exactly.
-            const int row = (int)(((uint32_t)loc * ((65535u + (uint32_t)w) / (uint32_t)w)) >> 16);
-            const int col = loc - row * w;
-            claim = tile_claim(q, true, x0 + col, y0 + row, tile, W, H);
+            const int row = (int)(((uint32_t)loc * (pw >> kPreBits & 0x1ffffu)) >> 16);
+            const int col = loc - row * ((int)(q.xs >> 16) - (int)(q.xs & 0xffffu) + 1);
+            const int tx = (int)(q.xs & 0xffffu) + col, ty = (int)(q.ys & 0xffffu) + row;
+            if (pw >> kFastBit) {
+                claim = tile_claim_div(
+                    q, tx, ty, tile, W, H,
+                    [&](float x) { return div_known(x, q.a, d.x, d.y); },
+                    [&](float x) { return div_known(x, q.c, d.z, d.w); });
+            } else {
+                claim = tile_claim(q, true, tx, ty, tile, W, H);
+            }
         }
         // The candidates of one rectangle in this round are a run of lanes
-        // starting at a head mark (or at lane 0); the run's first lane folds
-        // the run's claims into the rectangle's mask.
+        // starting at a head (or at lane 0); the run's first lane folds the
+        // run's claims into the rectangle's mask.
         const uint64_t cm = ballot(claim);
-        const uint64_t hm = ballot(valid && (h != 0 || lane == 0));
-        if (valid && (h != 0 || lane == 0)) {
+        if (valid && (head || lane == 0)) {
             const uint64_t above = lane == 63 ? 0ull : hm >> (lane + 1);
             const int len = above ? __builtin_ctzll(above) + 1 : min(64, total - c0) - lane;
             const uint32_t bits = (uint32_t)((cm >> lane) & ((len >= 64) ? ~0ull
                                                                           : ((1ull << len) - 1ull)));
-            w_msk[ol] |= bits << loc;
+            w_msk[own] |= bits << loc;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    return w_msk[lane];
+    return ar > 0 ? w_msk[rk] : 0u;
 }
 
 // Longest-processing-time-first orders, by one 1024-thread workgroup: a
@@ -762,8 +864,8 @@ bin_count_rec_kernel(const BinArgs A, int32_t *counts, BinRec *recs, uint32_t *m
     __shared__ BinRec s_rec[kBinThreads];
     __shared__ int32_t s_big[kBinThreads], s_cnt[kBinThreads];
     __shared__ int32_t s_nbig, s_used;
-    __shared__ int32_t s_pre[kBinThreads];
-    __shared__ uint32_t s_msk[kBinThreads];
+    __shared__ uint32_t s_pre[kBinThreads], s_msk[kBinThreads];
+    __shared__ float4 s_div[kBinThreads];
     // Per wave: the small claims' owner marks, then the strip walk's row
     // boundaries.
     __shared__ float4 s_rows[kBinThreads / 64][kRowSlots];
@@ -793,11 +895,11 @@ bin_count_rec_kernel(const BinArgs A, int32_t *counts, BinRec *recs, uint32_t *m
     // The claimed tiles of a small rectangle, bit loc for its row-major tile
     // loc: the write pass emits from them without testing again.
     mask = wave_small_claims(r, ar, test, A.tile, A.W, A.H, s_rec + wave * 64,
-                             s_pre + wave * 64, s_msk + wave * 64,
+                             s_div + wave * 64, s_pre + wave * 64, s_msk + wave * 64,
                              reinterpret_cast<uint8_t *>(s_rows[wave]), lane);
     n = __popc(mask);
-    // s_rec's wave slice now holds the big rectangles' records (a lane's own
-    // record, written by wave_small_claims or here).
+    // s_rec's wave slice, read to the end by its wave, now takes the big
+    // rectangles' records.
     if (big) s_rec[tid] = r;
     // Large rectangles: compacted in LDS, one wave each.
     const uint64_t m = ballot(big);
@@ -822,28 +924,25 @@ bin_count_rec_kernel(const BinArgs A, int32_t *counts, BinRec *recs, uint32_t *m
         int cnt = 0, t = 0;
         strip_walk(r, P, test, A.tile, A.W, A.H, s_rows[wave], lane,
                    [&](bool claim, int, int) {
-                       cnt += claim ? 1 : 0;
-                       if (keep) {
-                           const uint64_t cm = ballot(claim);
-                           if (lane == 0) wp[t] = cm;
-                       }
+                       const uint64_t cm = ballot(claim);
+                       cnt += __popcll(cm);
+                       if (keep && lane == 0) wp[t] = cm;
                        ++t;
                    });
-        for (int o = 32; o >= 1; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
         if (lane == 0) {
             s_cnt[j] = cnt;
-            s_pre[j] = (int32_t)(keep ? kept_mask(first, nst) : 0u);
+            s_pre[j] = keep ? kept_mask(first, nst, P.R) : 0u;
         }
     }
     __syncthreads();
     if (g < A.N) {
         if (big) n = s_cnt[tid];
         counts[g] = n;
-        masks[g] = big ? (uint32_t)s_pre[tid] : mask;
+        masks[g] = big ? s_pre[tid] : mask;
     }
-    unsigned long long tot = (unsigned long long)n;
-    for (int o = 32; o >= 1; o >>= 1) tot += __shfl_xor(tot, o, 64);
-    if ((threadIdx.x & 63) == 0) s_p[threadIdx.x >> 6] = BinPart{tot};
+    // Summed in halves, whose sums over a wave fit 32 bits.
+    const uint32_t lo = (uint32_t)wave_incl_sum(n & 0xffff), hi = (uint32_t)wave_incl_sum(n >> 16);
+    if (lane == 63) s_p[wave] = BinPart{lo + ((unsigned long long)hi << 16)};
     __syncthreads();
     if (threadIdx.x == 0) {
         BinPart b = s_p[0];
@@ -922,14 +1021,7 @@ constexpr int kBinStage = 2048;
 __device__ __forceinline__ void block_excl_sum_max(int vs, int vm, int &ex_s, int &ex_m,
                                                    int *sc) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int is = vs, im = vm;
-    for (int o = 1; o < 64; o <<= 1) {
-        const int ts = __shfl_up(is, o, 64), tm = __shfl_up(im, o, 64);
-        if (lane >= o) {
-            is += ts;
-            im = max(im, tm);
-        }
-    }
+    const int is = wave_incl_sum(vs), im = wave_incl_max(vm);
     if (lane == 63) {
         sc[wave] = is;
         sc[kBinThreads / 64 + wave] = im;
@@ -1039,6 +1131,14 @@ __global__ __launch_bounds__(kBinThreads) void bin_write_rec_kernel(
                     // Its run of words, marked at its start.
                     atomicMax(&s_wext, kept_first(mask) + kept_steps(mask));
                     s_hown[kept_first(mask)] = (uint16_t)(tid + 1);
+                    // The count pass's walk plan (strip_plan), from its rows a
+                    // step: R and s up to 64, ceil(2^16 / s) up to 2^16.
+                    const int R = kept_rows(mask);
+                    const int s = strip_cols((int)(r.xs >> 16) - (int)(r.xs & 0xffffu) + 1, R);
+                    s_pl[tid] = (uint32_t)R | (uint32_t)s << 7 |
+                                (uint32_t)small_ceil_div(65536, s) << 14;
+                    s_pnr[tid] =
+                        small_ceil_div((int)(r.ys >> 16) - (int)(r.ys & 0xffffu) + 1, R);
                 } else {
                     atomicAdd(&s_nfall, 1);
                 }
@@ -1053,14 +1153,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_write_rec_kernel(
     if (lane == 0 && m) slot = atomicAdd(&s_nbig, __popcll(m));
     slot = __shfl(slot, 0, 64);
     if (big) s_big[slot + rank_in(m)] = tid;
-    int incl = small_cap, cincl = cap;
-    for (int o = 1; o < 64; o <<= 1) {
-        const int t = __shfl_up(incl, o, 64), u = __shfl_up(cincl, o, 64);
-        if (lane >= o) {
-            incl += t;
-            cincl += u;
-        }
-    }
+    const int incl = wave_incl_sum(small_cap), cincl = wave_incl_sum(cap);
     if (lane == 63) {
         s_wsum[wave] = incl;
         s_csum[wave] = cincl;
@@ -1078,18 +1171,6 @@ __global__ __launch_bounds__(kBinThreads) void bin_write_rec_kernel(
     s_cap[tid] = cap;
     const int wext = s_wext, nbig = s_nbig;
     if (wext > 0) {   // workgroup-uniform
-        // The kept rectangles' walk plans, a wave each.
-        for (int e = wave; e < nbig; e += kBinThreads / 64) {
-            const int j = s_big[e];
-            if (s_wm[j] == 0) continue;
-            const StripPlan P = strip_plan(s_rec[j], lane);
-            if (lane == 0) {
-                // R and s up to 64, ceil(2^16 / s) up to 2^16.
-                s_pl[j] = (uint32_t)P.R | (uint32_t)P.s << 7 |
-                          ((65535u + (uint32_t)P.s) / (uint32_t)P.s) << 14;
-                s_pnr[j] = P.nr;
-            }
-        }
         // Words 4 tid .. 4 tid + 3, all requested at once.
         const int i0 = 4 * tid;
         uint64_t v[4];
@@ -1110,7 +1191,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_write_rec_kernel(
             psum += __popcll(v[q]);
         }
         int ex_s, ex_m;
-        block_excl_sum_max(psum, runmax, ex_s, ex_m, s_sc);   // orders the plans too
+        block_excl_sum_max(psum, runmax, ex_s, ex_m, s_sc);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int i = i0 + q;
@@ -1118,7 +1199,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_write_rec_kernel(
             const int st = max(hp[q], ex_m) - 1;      // the run's first word
             const int j = (int)s_hown[st] - 1;
             const int t = i - st, nr = s_pnr[j];
-            const int kk = t / nr, u = t - kk * nr;
+            const int kk = small_div(t, nr), u = t - kk * nr;
             const uint32_t pl = s_pl[j];
             const BinRec rj = s_rec[j];
             s_words[i] = v[q];
@@ -1186,7 +1267,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_write_rec_kernel(
             // loc < 32 <= 2^16 / w.
             const int x0 = (int)(r.xs & 0xffffu), y0 = (int)(r.ys & 0xffffu);
             const int w = (int)(r.xs >> 16) - x0 + 1;
-            const uint32_t inv = (65536u + (uint32_t)w - 1u) / (uint32_t)w;
+            const uint32_t inv = (uint32_t)small_ceil_div(65536, w);
             int n = 0;
             for (uint32_t mm = mask; mm != 0 && n < small_cap; mm &= mm - 1u, ++n) {
                 const int sl = first + n;

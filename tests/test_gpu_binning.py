@@ -168,6 +168,50 @@ def test_synthetic_conics_on_large_rectangles_bit_exact(dev, seed):
     assert np.array_equal(gids.cpu().numpy(), rids), "gauss_ids differ"
 
 
+@pytest.mark.parametrize("kind", ["ordinary", "wide_b", "tiny_centre", "wide_diagonal"])
+def test_small_rectangles_over_the_range_of_their_operands_bit_exact(dev, kind):
+    """Rectangles of 1 to about 100 tiles, whose tests share their Gaussian's
+    reciprocals where its conic and centre lie in a stated range and divide
+    where they do not: off-diagonals from denormal to 2^30, centres from
+    denormal up next to the image's zero edges, diagonals up to 2^40 and
+    significands of all ones. Exactly the oracle's lists."""
+    from metal_gauss_amd.backend import _bin
+
+    rng = np.random.default_rng(71)
+    N, W, H, tile = 6000, 640, 480, 16
+    f32 = np.float32
+    uv = np.stack([rng.uniform(0, W, N), rng.uniform(0, H, N)], 1).astype(f32)
+    rxy = rng.uniform(1, 90, (N, 2)).astype(f32)
+    a = np.exp(rng.uniform(np.log(1e-4), np.log(1.0), N)).astype(f32)
+    c = np.exp(rng.uniform(np.log(1e-4), np.log(1.0), N)).astype(f32)
+    b = (rng.uniform(-0.999, 0.999, N) * np.sqrt(a.astype(np.float64) * c)).astype(f32)
+    ones = rng.random(N) < 0.2      # significands of all ones, but for the last bits
+    for x in (a, c):
+        x.view(np.uint32)[ones] |= np.uint32(0x7FFFF8)
+    if kind == "wide_b":
+        b = (np.sign(b) * np.exp2(rng.uniform(-149, 30, N))).astype(f32)
+        b[rng.random(N) < 0.2] = 0.0
+    elif kind == "tiny_centre":
+        near = rng.random(N) < 0.7
+        uv[near, 0] = (np.exp2(rng.uniform(-149, 0, near.sum()))).astype(f32)
+        near = rng.random(N) < 0.7
+        uv[near, 1] = (-np.exp2(rng.uniform(-149, 0, near.sum()))).astype(f32)
+    elif kind == "wide_diagonal":
+        a *= np.exp2(rng.uniform(-40, 40, N)).astype(f32)
+        c *= np.exp2(rng.uniform(-40, 40, N)).astype(f32)
+    conic = np.stack([a, b, c], 1).astype(f32)
+    op = rng.uniform(0.05, 0.99, N).astype(f32)
+    valid = np.ones(N, np.int32)
+    depth = rng.uniform(0.5, 20.0, N).astype(f32)
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(dev)
+    gids, offs, _ = _bin(t(uv), t(rxy), t(depth), t(valid), t(conic), t(op), W, H, tile)
+    rids, roffs, _, _ = binning_ref.build_tile_lists(uv, rxy, conic, op, valid, depth, W, H,
+                                                     tile, ellipse=True)
+    assert rids.size > N
+    assert np.array_equal(offs.cpu().numpy(), roffs), "tile offsets differ"
+    assert np.array_equal(gids.cpu().numpy(), rids), "gauss_ids differ"
+
+
 @pytest.mark.parametrize("ellipse", [True, False])
 def test_kept_and_rewalked_large_rectangles_bit_exact(dev, ellipse):
     """The count pass keeps a large rectangle's claims as one 64-bit word per
