@@ -247,10 +247,14 @@ __device__ __forceinline__ bool tile_claim(const BinRec &r, bool test, int tx, i
         [&](float x) { return x / r.c; });
 }
 
-// Rectangles larger than this many tiles are walked by a whole wave instead
-// of one thread: near-camera Gaussians can cover thousands of tiles, and one
-// thread walking them holds up its workgroup.
-constexpr int kWaveWalkArea = 32;
+// Rectangles of up to kWaveWalkArea tiles are tested one candidate tile a lane
+// (wave_small_claims), larger ones are walked by a whole wave each: a walk
+// takes about 240 instructions before its steps, 64 candidates 130, and a
+// claim mask has 64 bits. Up to kMaskArea tiles the mask is one of the mask
+// words; above, it is a kept word (see kept_mask). With the line at 32 tiles
+// the count pass took 32 us instead of 29.5 at 600k Gaussians (15k rectangles
+// of 33 to 64 tiles), 290 instead of 243 at 3.6M crowded ones (275k of them).
+constexpr int kMaskArea = 32, kWaveWalkArea = 64;
 
 // A wave's walk of one large rectangle, lanes on fixed columns. The
 // rectangle is cut into strips of s columns; a step covers R rows of a strip
@@ -273,7 +277,6 @@ constexpr int kWaveWalkArea = 32;
 // order: a Gaussian's pairs go to distinct tiles, so their order within its
 // run does not reach the sorted tile lists.
 constexpr int kRowSlots = 128;
-static_assert(kRowSlots * 16 == 64 * kWaveWalkArea, "the row slice aliases the small-claim bytes");
 
 // The shape of a wave's walk over one large rectangle: ns strips of s
 // columns, each nr steps of R rows; lane = row group rg * s + column cl.
@@ -663,8 +666,8 @@ __device__ __forceinline__ int wave_incl_sum(int v) {
 // candidate per lane: a per-lane walk made every lane wait for the wave's
 // largest rectangle. Lane l's rectangle has ar tiles (0 for none); the
 // rectangles that have any lie in lane order in the wave's slices, one's
-// candidates are [pre, pre + ar) of the wave's row with a mark at the first,
-// and a candidate's rectangle is the number of marks up to it. What a
+// candidates are [pre, pre + ar) of the wave's row with a mark bit at the
+// first, and a candidate's rectangle is the number of marks up to it. What a
 // candidate would divide by is a property of its rectangle and formed once
 // for it: the reciprocals of a and c (ClaimDiv) and of the width. The test is
 // arithmetic-bound, and dividing per candidate took about a third of it
@@ -672,22 +675,23 @@ __device__ __forceinline__ int wave_incl_sum(int v) {
 // Each tile's decision is tile_claim's, the walk's own expressions, so the
 // result is bit for bit the walk's. Returns this lane's claim mask (bit loc
 // for tile loc).
-constexpr int kPreBits = 11, kFastBit = 28;
+constexpr int kPreBits = 12, kFastBit = 29;
 static_assert(63 * kWaveWalkArea < (1 << kPreBits), "pre fits below the width's reciprocal");
+static_assert(64 * kWaveWalkArea / 8 <= 16 * kRowSlots, "the marks fit a row slice");
 
-__device__ __forceinline__ uint32_t wave_small_claims(const BinRec &r, int ar, bool test,
+__device__ __forceinline__ uint64_t wave_small_claims(const BinRec &r, int ar, bool test,
                                                       int tile, int W, int H, BinRec *w_rec,
                                                       float4 *w_div, uint32_t *w_pre,
-                                                      uint32_t *w_msk, uint8_t *w_own,
+                                                      uint64_t *w_msk, uint64_t *w_mark,
                                                       int lane) {
-    if (!test) return ar >= 32 ? 0xFFFFFFFFu : (1u << ar) - 1u;
+    if (!test) return ar >= 64 ? ~0ull : (1ull << ar) - 1ull;
     const int incl = wave_incl_sum(ar);
     const int pre = incl - ar;
     const int total = __builtin_amdgcn_readlane(incl, 63);
-    if (total == 0) return 0u;   // wave-uniform
+    if (total == 0) return 0ull;   // wave-uniform
     const int rk = rank_in(ballot(ar > 0));
     if (ar > 0) {
-        // loc < 32 and w <= 32: loc * ceil(2^16 / w) >> 16 is loc / w exactly.
+        // loc < 64 and w <= 64: loc * ceil(2^16 / w) >> 16 is loc / w exactly.
         const int w = (int)(r.xs >> 16) - (int)(r.xs & 0xffffu) + 1;
         const uint32_t inv = (uint32_t)small_ceil_div(65536, w);
         const ClaimDiv d = claim_div(r);
@@ -695,13 +699,13 @@ __device__ __forceinline__ uint32_t wave_small_claims(const BinRec &r, int ar, b
         w_div[rk] = make_float4(d.ia, d.ia_lo, d.ic, d.ic_lo);
         w_pre[rk] = (uint32_t)pre | inv << kPreBits |
                     (quotients_safe(r) ? 1u << kFastBit : 0u);
-        w_msk[rk] = 0u;
+        w_msk[rk] = 0ull;
     }
-    for (int i = lane; i < (total + 3) / 4; i += 64) reinterpret_cast<uint32_t *>(w_own)[i] = 0u;
+    w_mark[lane] = 0ull;   // 64 bits for each of up to kWaveWalkArea rounds
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (ar > 0) w_own[pre] = (uint8_t)1;
+    if (ar > 0) atomicOr(reinterpret_cast<uint32_t *>(w_mark) + (pre >> 5), 1u << (pre & 31));
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -709,8 +713,8 @@ __device__ __forceinline__ uint32_t wave_small_claims(const BinRec &r, int ar, b
     for (int c0 = 0; c0 < total; c0 += 64) {
         const int c = c0 + lane;
         const bool valid = c < total;
-        const bool head = valid && w_own[c] != 0;
-        const uint64_t hm = ballot(head);
+        const uint64_t hm = w_mark[c0 >> 6];
+        const bool head = (hm >> lane) & 1ull;
         // The first candidate is a head, so own >= 0.
         const int own = before + rank_in(hm) + (head ? 1 : 0);
         before += __popcll(hm);
@@ -739,15 +743,14 @@ __device__ __forceinline__ uint32_t wave_small_claims(const BinRec &r, int ar, b
         if (valid && (head || lane == 0)) {
             const uint64_t above = lane == 63 ? 0ull : hm >> (lane + 1);
             const int len = above ? __builtin_ctzll(above) + 1 : min(64, total - c0) - lane;
-            const uint32_t bits = (uint32_t)((cm >> lane) & ((len >= 64) ? ~0ull
-                                                                          : ((1ull << len) - 1ull)));
+            const uint64_t bits = (cm >> lane) & (len >= 64 ? ~0ull : (1ull << len) - 1ull);
             w_msk[own] |= bits << loc;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    return ar > 0 ? w_msk[rk] : 0u;
+    return ar > 0 ? w_msk[rk] : 0ull;
 }
 
 // Longest-processing-time-first orders, by one 1024-thread workgroup: a
@@ -864,7 +867,8 @@ bin_count_rec_kernel(const BinArgs A, int32_t *counts, BinRec *recs, uint32_t *m
     __shared__ BinRec s_rec[kBinThreads];
     __shared__ int32_t s_big[kBinThreads], s_cnt[kBinThreads];
     __shared__ int32_t s_nbig, s_used;
-    __shared__ uint32_t s_pre[kBinThreads], s_msk[kBinThreads];
+    __shared__ uint32_t s_pre[kBinThreads];
+    __shared__ uint64_t s_msk[kBinThreads];
     __shared__ float4 s_div[kBinThreads];
     // Per wave: the small claims' owner marks, then the strip walk's row
     // boundaries.
@@ -881,7 +885,7 @@ bin_count_rec_kernel(const BinArgs A, int32_t *counts, BinRec *recs, uint32_t *m
     __syncthreads();
     int n = 0;
     bool big = false;
-    uint32_t mask = 0;
+    uint64_t claims = 0;
     BinRec r{};
     int ar = 0;
     if (g < A.N && make_rec(A, g, r)) {
@@ -894,10 +898,26 @@ bin_count_rec_kernel(const BinArgs A, int32_t *counts, BinRec *recs, uint32_t *m
     }
     // The claimed tiles of a small rectangle, bit loc for its row-major tile
     // loc: the write pass emits from them without testing again.
-    mask = wave_small_claims(r, ar, test, A.tile, A.W, A.H, s_rec + wave * 64,
+    claims = wave_small_claims(r, ar, test, A.tile, A.W, A.H, s_rec + wave * 64,
                              s_div + wave * 64, s_pre + wave * 64, s_msk + wave * 64,
-                             reinterpret_cast<uint8_t *>(s_rows[wave]), lane);
-    n = __popc(mask);
+                             reinterpret_cast<uint64_t *>(s_rows[wave]), lane);
+    n = __popcll(claims);
+    uint32_t mask = (uint32_t)claims;
+    // Past kMaskArea tiles the claims are one kept word, that of a walk whose
+    // single step has all the rectangle's rows: its lanes are the row-major
+    // tiles. Taken before the walks' words, at most one a thread: they fit.
+    {
+        static_assert(kBinThreads <= kBlockWords, "a word for every thread");
+        const bool word = ar > kMaskArea;
+        const uint64_t m = ballot(word);
+        int at = 0;
+        if (lane == 0 && m) at = atomicAdd(&s_used, __popcll(m));
+        at = __builtin_amdgcn_readfirstlane(at) + rank_in(m);
+        if (word) {
+            words[blk * kBlockWords + at] = claims;
+            mask = kept_mask(at, 1, (int)(r.ys >> 16) - (int)(r.ys & 0xffffu) + 1);
+        }
+    }
     // s_rec's wave slice, read to the end by its wave, now takes the big
     // rectangles' records.
     if (big) s_rec[tid] = r;
@@ -1046,7 +1066,7 @@ __device__ __forceinline__ void block_excl_sum_max(int vs, int vm, int &ex_s, in
 //     256 x 32 pairs) and staged in windows of kBinStage slots, each slot
 //     with its position in the range, then stored by consecutive lanes, so
 //     adjacent runs land as coalesced stores.
-//   * Large rectangles (more than kWaveWalkArea tiles) are replayed from the
+//   * Large rectangles (more than kMaskArea tiles) are replayed from the
 //     step words the count pass kept. Those words are one run per rectangle
 //     from the start of the workgroup's kBlockWords. The workgroup loads
 //     them, finds each word's rectangle (the last run start at or before it,
@@ -1122,7 +1142,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_write_rec_kernel(
             g = (int32_t)k;
             r = recs[g];
             mask = masks[g];
-            if (rec_area(r) > kWaveWalkArea) {
+            if (rec_area(r) > kMaskArea) {
                 big = true;
                 s_rec[tid] = r;
                 s_g[tid] = g;
@@ -1226,17 +1246,35 @@ __global__ __launch_bounds__(kBinThreads) void bin_write_rec_kernel(
                 ids[at] = s_g[j];
         }
     };
-    // The kept words, the four waves in turn.
-    for (int i = wave; i < wext; i += kBinThreads / 64) {
-        const uint64_t cm = s_words[i];
-        if (cm == 0) continue;
-        const int j = (int)s_hown[i] - 1;
-        const uint32_t tb = s_tb[i], pl = s_pl[j];
-        // lane = rg * s + cl, rg = floor(lane / s) as lane * ceil(2^16 / s) >> 16
-        // (exact for lane < 64 <= 2^16 / s).
-        const int sw = (int)((pl >> 7) & 127u);
-        const int rg = (int)(((uint32_t)lane * (pl >> 14)) >> 16), cl = lane - rg * sw;
-        emit(cm, j, (int)(tb & 0xffffu) + cl, (int)(tb >> 16) + rg, s_pw[i] - s_pf[j]);
+    // The kept words, the four waves in turn, kEmit words a wave at a time:
+    // a word's LDS reads depend on one another, several words' do not (1.5M
+    // words: 228 us one at a time, 221 so).
+    constexpr int kEmit = 4, kEmitStep = kEmit * (kBinThreads / 64);
+    for (int i0 = wave * kEmit; i0 < wext; i0 += kEmitStep) {
+        uint64_t cm[kEmit];
+        int j[kEmit], pos[kEmit];
+        uint32_t tb[kEmit], pl[kEmit];
+#pragma unroll
+        for (int q = 0; q < kEmit; ++q) {
+            const int i = min(i0 + q, wext - 1);
+            cm[q] = i0 + q < wext ? s_words[i] : 0ull;
+            j[q] = (int)s_hown[i] - 1;
+            tb[q] = s_tb[i];
+            pos[q] = s_pw[i];
+        }
+#pragma unroll
+        for (int q = 0; q < kEmit; ++q) {
+            pl[q] = s_pl[j[q]];
+            pos[q] -= s_pf[j[q]];
+        }
+#pragma unroll
+        for (int q = 0; q < kEmit; ++q) {
+            // lane = rg * s + cl, rg = floor(lane / s) as lane * ceil(2^16 / s) >> 16
+            // (exact for lane < 64 <= 2^16 / s).
+            const int sw = (int)((pl[q] >> 7) & 127u);
+            const int rg = (int)(((uint32_t)lane * (pl[q] >> 14)) >> 16), cl = lane - rg * sw;
+            emit(cm[q], j[q], (int)(tb[q] & 0xffffu) + cl, (int)(tb[q] >> 16) + rg, pos[q]);
+        }
     }
     // Rectangles without kept words: walked again, a wave each, in the row
     // slices (s_k, once the replay is done with it).

@@ -213,6 +213,46 @@ def test_small_rectangles_over_the_range_of_their_operands_bit_exact(dev, kind):
 
 
 @pytest.mark.parametrize("ellipse", [True, False])
+@pytest.mark.parametrize("shape", [(4, 8), (32, 1), (3, 11), (8, 8), (64, 1), (1, 64), (5, 13)])
+def test_rectangles_of_every_mask_size_bit_exact(dev, shape, ellipse):
+    """The claims of up to 32 tiles are one mask word, of up to 64 a kept
+    64-bit word, of more the kept words of a walk. Two blocks of Gaussians that
+    all have one rectangle size at those edges (every thread takes a word, a
+    wave has 64 rounds of candidates), then one that mixes it with rectangles
+    of over a thousand tiles, whose walks take the words that are left.
+    Exactly the oracle's lists."""
+    from metal_gauss_amd.backend import _bin
+
+    w, h = shape
+    rng = np.random.default_rng(73)
+    N, W, H, tile = 768, 1120, 1120, 16
+    f32 = np.float32
+    half = np.array([w, h]) * tile / 2
+    # Within a quarter tile of w x h whole tiles' middle, the extent as much less.
+    first = np.stack([rng.integers(0, W // tile - w + 1, N), rng.integers(0, H // tile - h + 1, N)], 1)
+    uv = (first * tile + half + rng.uniform(-3, 3, (N, 2))).astype(f32)
+    rxy = np.broadcast_to(half - 4, (N, 2)).astype(f32).copy()
+    wide = 512 + np.arange(0, 256, 5)
+    rxy[wide] = rng.uniform(300, 700, (wide.size, 2))
+    sig = rxy / 3.0
+    corr = rng.uniform(-0.95, 0.95, N)
+    a, c = 1 / (sig[:, 0] ** 2 * (1 - corr**2)), 1 / (sig[:, 1] ** 2 * (1 - corr**2))
+    conic = np.stack([a, -corr * np.sqrt(a * c), c], 1).astype(f32)
+    op = rng.uniform(0.05, 0.99, N).astype(f32)
+    valid = np.ones(N, np.int32)
+    depth = rng.uniform(0.5, 20.0, N).astype(f32)
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(dev)
+    cn, o = (t(conic), t(op)) if ellipse else (None, None)
+    gids, offs, _ = _bin(t(uv), t(rxy), t(depth), t(valid), cn, o, W, H, tile)
+    rids, roffs, _, _ = binning_ref.build_tile_lists(uv, rxy, conic, op, valid, depth, W, H,
+                                                     tile, ellipse=ellipse)
+    if not ellipse:
+        assert (np.bincount(rids, minlength=N)[:512] == w * h).all()
+    assert np.array_equal(offs.cpu().numpy(), roffs), "tile offsets differ"
+    assert np.array_equal(gids.cpu().numpy(), rids), "gauss_ids differ"
+
+
+@pytest.mark.parametrize("ellipse", [True, False])
 def test_kept_and_rewalked_large_rectangles_bit_exact(dev, ellipse):
     """The count pass keeps a large rectangle's claims as one 64-bit word per
     walk step, up to 256 words per wave of its workgroup, and the write pass
