@@ -1382,25 +1382,24 @@ inline int tile_bits(int n_tiles) {
 //   3. count_scatter - each workgroup holds its chunk in registers, one
 //                      contiguous part of 64 * per pairs per wave, counts
 //                      each part into a wave-private LDS histogram, forms the
-//                      tile starts (exclusive scan of the totals) and from
-//                      them each wave's first slot per tile, then walks its
-//                      part in input order, ranking pairs of one tile by
-//                      ballots over the tile bits, and stores each id at its
-//                      slot.
+//                      tile starts (exclusive scan of the totals) and each
+//                      wave's first slot per tile, then walks its part in
+//                      input order, ranking pairs of one tile by ballots over
+//                      the tile bits; the chunk is put in tile order through
+//                      LDS and stored.
 // A pair's slot is start(t) + the pairs of tile t in earlier chunks, in
 // earlier waves' parts and earlier in its own part: the input order within
 // each tile, i.e. the stable order. The tile starts double as the list
 // offsets. Pairs with a tile >= n_tiles are dropped.
 constexpr int kCsBuckets = 4096;
 constexpr int kCsThreads = 256, kCsWaves = kCsThreads / 64;
-constexpr int64_t kCsMaxChunks = 512;   // about two workgroups per CU
+constexpr int64_t kCsMaxChunks = 768;   // three workgroups per CU
 // Capacity-bounded lists plan for the capacity, which runs above the pairs
-// actually sorted (by the caller's headroom, or more). With twice the limit
-// the kept pairs get chunks no longer than the exact plan's as long as the
-// capacity is at most twice their count; with the same limit a headroom that
-// crossed it would lengthen the chunks a step and leave part of the GPU idle
-// (measured: 94 -> 113 us at config 4).
-constexpr int64_t kCsMaxChunksCapped = 2 * kCsMaxChunks;
+// actually sorted (by the caller's headroom, or more). At the default
+// headroom of a quarter the kept pairs of a full plan are 1024 chunks, what
+// the column scan holds at once; with the exact limit a headroom that crossed
+// it would lengthen the chunks a step and leave part of the GPU idle.
+constexpr int64_t kCsMaxChunksCapped = 1280;
 constexpr int kColWaves = 16;           // waves of the column scan's workgroups
 
 struct CsPlan {
@@ -1408,9 +1407,12 @@ struct CsPlan {
     int64_t nchunks;
 };
 
-// The smallest chunk that needs no more than max_chunks workgroups.
+// The smallest chunk that needs no more than max_chunks workgroups. 24 pairs a
+// lane keep three workgroups on a CU; 16 and 32 were worse wherever they lay
+// next to it (3.6M pairs over 4056 tiles: 48 us with 16, 40 with 24; 5.1M over
+// 2500: 75 with 32, whose registers leave two workgroups a CU, 59 with 24).
 inline CsPlan cs_plan(int64_t n, int64_t max_chunks = kCsMaxChunks) {
-    static const int kPers[] = {8, 16, 24, 32, 48, 64};
+    static const int kPers[] = {8, 24, 48, 64};
     for (int p : kPers) {
         const int64_t nc = ceil_div(n, (int64_t)kCsThreads * p);
         if (nc <= max_chunks || p == 64) return {p, nc};
@@ -1596,12 +1598,7 @@ __device__ __forceinline__ void cs_depth_order(const CsPass<V> &P, uint32_t *s_w
     const int nb = P.nb, t0 = tid * kTPer;
 
     // A counting sort of the tiles over 256 list-length bins (tiles of one
-    // bin in no fixed order), in the LDS of the scatter's wave counters.
-    if (nb < kCsThreads / kCsWaves) {
-        // Fewer words of wave counters than bins: the tiles in order.
-        for (int i = tid; i < nb; i += kCsThreads) P.order[i] = i;
-        return;
-    }
+    // bin in no fixed order), in the scatter's LDS.
     uint32_t *hb = s_wh;   // kCsThreads bins
     hb[tid] = 0;
     __syncthreads();
@@ -1634,19 +1631,30 @@ __device__ __forceinline__ void cs_depth_order(const CsPass<V> &P, uint32_t *s_w
         if (bin[j] >= 0) P.order[hb[bin[j]] + slot[j]] = t0 + j;
 }
 
+// LDS of the scatter. Until the ranks are known: per wave and tile a 16-bit
+// count, then local slot (rows of an even number of tiles), and per tile the
+// distance from a local slot to its slot in the output. Then a window of the
+// chunk's pairs in local order, each with its slot.
+template <int kPer>
+constexpr int cs_window() { return kPer % 12 == 0 ? 3072 : 2048; }
+template <int kPer, typename V>
+inline unsigned cs_scatter_lds(int nb) {
+    return (unsigned)std::max(2 * kCsWaves * ((nb + 1) & ~1) + 4 * nb,
+                              cs_window<kPer>() * (4 + (int)sizeof(V)));
+}
+
 template <int kPer, typename V>
 __global__ __launch_bounds__(kCsThreads) void count_scatter_kernel(const CsPass<V> P) {
     constexpr int64_t kChunk = (int64_t)kCsThreads * kPer, kPart = 64 * kPer;
-    constexpr int kTPer = kCsBuckets / kCsThreads;   // tiles owned per thread
-    // Per wave and tile: the count, then the next slot; sized by the launch
-    // to the tile count (kCsWaves * nb words), so that at config 4's 2500
-    // tiles four workgroups share a CU and every chunk's workgroup is
-    // resident at once (two with room for 4096 tiles).
-    extern __shared__ uint32_t s_wh[];
-    __shared__ uint32_t s_part[kCsWaves];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int kTPer = kCsBuckets / kCsThreads + 1;   // tiles owned per thread, at most
+    constexpr int kWin = cs_window<kPer>();
+    static_assert(kChunk % kWin == 0 && kWin % kCsThreads == 0, "whole windows");
+    extern __shared__ __align__(16) uint32_t s_mem[];
+    __shared__ uint32_t s_part[2 * kCsWaves];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (P.order && blockIdx.x == gridDim.x - 1) {   // the depth sort's order
-        cs_depth_order(P, s_wh, s_part);
+        cs_depth_order(P, s_mem, s_part);
         return;
     }
     const int64_t n = cs_count(P);
@@ -1654,59 +1662,80 @@ __global__ __launch_bounds__(kCsThreads) void count_scatter_kernel(const CsPass<
     if ((int64_t)blockIdx.x >= nact) return;
     const int64_t c = xcd_contiguous(blockIdx.x, nact);
     const int64_t pb = c * kChunk + wave * kPart;
-    const int nb = P.nb;
+    const int left = (int)min(max(n - pb, (int64_t)0), kPart);   // pairs of the wave's part
+    const int nb = P.nb, nbe = (nb + 1) & ~1;
+    uint16_t *const s_wh = reinterpret_cast<uint16_t *>(s_mem);
+    uint32_t *const s_delta = s_mem + kCsWaves * nbe / 2;
     // The wave's part: pair pb + 64 r + lane is (tile t[r], id v[r]); a tile
     // of nb or more marks a dropped or absent pair.
     uint32_t t[kPer];
-    V v[kPer];
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
-        const int64_t i = pb + 64 * r + lane;
-        t[r] = i < n ? P.tiles[i] : 0xFFFFFFFFu;
-        v[r] = i < n ? P.ids[i] : V{};
+        const int i = 64 * r + lane;
+        t[r] = i < left ? (P.tiles + pb)[i] : 0xFFFFFFFFu;
     }
-    // Thread tid owns tiles [tid * kTPer, tid * kTPer + kTPer): their totals
-    // and this chunk's prefix, requested with the pairs.
-    const int t0 = tid * kTPer;
+    // Thread tid owns tiles [tid * tper, tid * tper + tper): their totals and
+    // this chunk's prefix, requested with the pairs (every load in range, its
+    // value used only where the tile exists, so no branch separates them).
+    // tper is odd, which spreads the lanes' LDS words at one tile of theirs
+    // over the banks (16 apart, four banks served all 64 lanes).
+    const int tper = ((nb + kCsThreads - 1) / kCsThreads) | 1;
+    const int t0 = tid * tper;
     uint32_t tv[kTPer], hv[kTPer];
 #pragma unroll
     for (int j = 0; j < kTPer; ++j) {
-        const bool in = t0 + j < nb;
-        tv[j] = in ? P.tot[t0 + j] : 0u;
-        hv[j] = in ? P.hist[c * nb + t0 + j] : 0u;
+        const int tt = min(t0 + j, nb - 1);
+        tv[j] = P.tot[tt];
+        hv[j] = P.hist[c * nb + tt];
     }
-    for (int i = tid; i < nb; i += kCsThreads) {
-#pragma unroll
-        for (int w = 0; w < kCsWaves; ++w) s_wh[w * nb + i] = 0;
-    }
+    for (int i = tid; i < kCsWaves * nbe / 2; i += kCsThreads) s_mem[i] = 0;
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kPer; ++r)
-        if (t[r] < (uint32_t)nb) atomicAdd(&s_wh[wave * nb + t[r]], 1u);
-    __syncthreads();
-    uint32_t sum = 0;
-#pragma unroll
-    for (int j = 0; j < kTPer; ++j) sum += tv[j];
-    uint32_t incl = sum;
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t u = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += u;
+    for (int r = 0; r < kPer; ++r) {
+        // Two counts a word; neither half can overflow (static_assert above).
+        const uint32_t i = (uint32_t)(wave * nbe) + t[r];
+        if (t[r] < (uint32_t)nb) atomicAdd(&s_mem[i >> 1], 1u << (16 * (i & 1)));
     }
-    if (lane == 63) s_part[wave] = incl;
     __syncthreads();
-    uint32_t start = incl - sum;
-    for (int w = 0; w < wave; ++w) start += s_part[w];
+    // Two exclusive scans over the tiles: the totals' (the tile starts) and
+    // the chunk's own counts' (the local starts).
+    uint32_t sum = 0, lsum = 0;
+#pragma unroll
+    for (int j = 0; j < kTPer; ++j) {
+        const bool in = j < tper && t0 + j < nb;
+        tv[j] = in ? tv[j] : 0u;
+        sum += tv[j];
+        if (in) {
+#pragma unroll
+            for (int w = 0; w < kCsWaves; ++w) lsum += s_wh[w * nbe + t0 + j];
+        }
+    }
+    const uint32_t incl = (uint32_t)wave_incl_sum((int)sum);
+    const uint32_t lincl = (uint32_t)wave_incl_sum((int)lsum);
+    if (lane == 63) {
+        s_part[wave] = incl;
+        s_part[kCsWaves + wave] = lincl;
+    }
+    __syncthreads();
+    uint32_t start = incl - sum, lstart = lincl - lsum;
+    int held = 0;   // pairs of this chunk that are kept
+#pragma unroll
+    for (int w = 0; w < kCsWaves; ++w) {
+        start += w < wave ? s_part[w] : 0u;
+        lstart += w < wave ? s_part[kCsWaves + w] : 0u;
+        held += (int)s_part[kCsWaves + w];
+    }
 #pragma unroll
     for (int j = 0; j < kTPer; ++j) {
         const int tt = t0 + j;
-        if (tt < nb) {
+        if (j < tper && tt < nb) {
             if (c == 0) P.offsets[tt] = (int32_t)start;
-            uint32_t slot = start + hv[j];
+            s_delta[tt] = start + hv[j] - lstart;
 #pragma unroll
             for (int w = 0; w < kCsWaves; ++w) {
-                const uint32_t cnt = s_wh[w * nb + tt];
-                s_wh[w * nb + tt] = slot;
-                slot += cnt;
+                const uint32_t cnt = s_wh[w * nbe + tt];
+                s_wh[w * nbe + tt] = (uint16_t)lstart;
+                lstart += cnt;
             }
         }
         start += tv[j];
@@ -1715,7 +1744,7 @@ __global__ __launch_bounds__(kCsThreads) void count_scatter_kernel(const CsPass<
     if (c == 0 && tid == kCsThreads - 1) P.offsets[nb] = (int32_t)start;
     __syncthreads();
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    uint32_t *wh = s_wh + wave * nb;
+    uint16_t *wh = s_wh + wave * nbe;
     // Lanes whose pair is in the same tile (kept pairs only): one ballot per
     // tile bit, kept where the bit agrees; x is -1 where this lane's bit is 0.
     auto peers_of = [&](uint32_t tt) {
@@ -1727,24 +1756,66 @@ __global__ __launch_bounds__(kCsThreads) void count_scatter_kernel(const CsPass<
         }
         return pm;
     };
+    // The values, in flight while the pairs are ranked.
+    V v[kPer];
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+        const int i = 64 * r + lane;
+        v[r] = i < left ? (P.ids + pb)[i] : V{};
+    }
     uint64_t next = peers_of(t[0]);
+    // Two local slots a word (0xFFFF: none; a chunk's are below 2^14 + 1); t
+    // becomes the slot in the output.
+    uint32_t lp[kPer / 2];
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
         const bool ok = t[r] < (uint32_t)nb;
         const uint64_t peers = next;
         const uint32_t wr = (uint32_t)__popcll(peers & lt);
         const uint32_t prior = ok ? wh[t[r]] : 0u;
-        // The next round's ballots overlap this round's LDS read.
+        const uint32_t delta = ok ? s_delta[t[r]] : 0u;
+        // The next round's ballots overlap this round's LDS reads.
         if (r + 1 < kPer) next = peers_of(t[r + 1]);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (ok && wr == 0) wh[t[r]] = prior + (uint32_t)__popcll(peers);
+        if (ok && wr == 0) wh[t[r]] = (uint16_t)(prior + (uint32_t)__popcll(peers));
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const uint32_t pos = prior + wr;
-        if (ok && (int64_t)pos < n) P.out[pos] = v[r];
+        const uint32_t slot = ok ? prior + wr : 0xFFFFu;
+        lp[r / 2] = r % 2 == 0 ? slot : lp[r / 2] | slot << 16;
+        t[r] = slot + delta;
+    }
+    // The chunk in local order, a window at a time, through LDS: every
+    // workgroup then writes its tiles in the same order at about the same
+    // time, so the lines that chunks share are completed in L2. Written in
+    // input order they left it in parts, 4.4 bytes a byte of output (now 1.1):
+    // 67 -> 40 us at 3.6M pairs over 4056 tiles, 70 -> 59 at 5.1M over 2500,
+    // 27 -> 21 at 1.5M.
+    V *const ex_v = reinterpret_cast<V *>(s_mem);
+    uint32_t *const ex_d = reinterpret_cast<uint32_t *>(ex_v + kWin);
+    for (int w0 = 0; w0 < held; w0 += kWin) {
+        // The tables, or the last window, are read out.
+        lds_reads_done();
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kPer; ++r) {
+            const uint32_t i = (lp[r / 2] >> (16 * (r % 2)) & 0xFFFFu) - (uint32_t)w0;
+            if (i < (uint32_t)kWin) {
+                ex_v[i] = v[r];
+                ex_d[i] = t[r];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kWin / kCsThreads; ++j) {
+            const int i = tid + kCsThreads * j;
+            if (w0 + i < held) {
+                const uint32_t pos = ex_d[i];
+                if ((int64_t)pos < n) P.out[pos] = ex_v[i];
+            }
+        }
     }
 }
 
@@ -1790,14 +1861,12 @@ static int32_t tile_count_sort(const uint32_t *tiles, const V *ids, int64_t n, i
             P, plan.nchunks);                                                          \
         MG_LAUNCHED("count_colscan_kernel");                                           \
         count_scatter_kernel<PER, V><<<grid + (P.order ? 1 : 0), kCsThreads,             \
-                                       4 * kCsWaves * n_tiles, s>>>(P);                   \
+                                       cs_scatter_lds<PER, V>(n_tiles), s>>>(P);          \
         MG_LAUNCHED("count_scatter_kernel");                                           \
         break;
     switch (plan.per) {
         MG_CS(8)
-        MG_CS(16)
         MG_CS(24)
-        MG_CS(32)
         MG_CS(48)
         MG_CS(64)
         default: MG_REQUIRE(false, "tile sort: %d pairs per lane", plan.per);

@@ -601,6 +601,35 @@ def test_sort_pairs_by_tile_is_stable_and_exact(dev, n, n_tiles, kind):
     assert (got[order.size:] == -1).all(), "wrote past the kept pairs"
 
 
+@pytest.mark.parametrize("n_tiles", [1, 2, 63, 255, 257, 2501, 4095, 4096])
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 1_600_000, 1_578_241, 4_800_003])
+def test_sort_pairs_by_tile_at_the_edges_of_its_windows(dev, n, n_tiles):
+    """Chunks of 2048, 6144 and 12288 pairs leave through LDS windows of 2048
+    or 3072; the last chunk holds one pair, a whole window, or part of one, and
+    a tenth of the pairs is dropped, so windows end anywhere. Even and odd
+    tile counts (the counters are two to a word), up to the most."""
+    from metal_gauss_amd import _lib
+
+    lib = _lib.load()
+    g = torch.Generator(device=dev).manual_seed(n + n_tiles)
+    tiles = torch.randint(0, n_tiles, (n,), generator=g, device=dev, dtype=torch.int32)
+    tiles[torch.rand(n, generator=g, device=dev) < 0.1] = n_tiles + 5
+    ids = torch.arange(n, dtype=torch.int32, device=dev).flip(0)
+    kept = tiles[tiles < n_tiles]
+    order = torch.sort(tiles, stable=True)[1][:kept.numel()]
+    counts = torch.bincount(kept.long(), minlength=n_tiles)
+    out = torch.full((n,), -1, dtype=torch.int32, device=dev)
+    offs = torch.full((n_tiles + 1,), -1, dtype=torch.int32, device=dev)
+    ws = torch.empty(lib.mg_sort_pairs_by_tile_workspace_bytes(n, n_tiles), dtype=torch.uint8,
+                     device=dev)
+    _lib.check(lib.mg_sort_pairs_by_tile(n, tiles.data_ptr(), ids.data_ptr(), n_tiles,
+                                         out.data_ptr(), offs.data_ptr(), ws.data_ptr(),
+                                         ws.numel(), _lib.stream(tiles)))
+    assert offs[0].item() == 0 and torch.equal(offs[1:].long(), counts.cumsum(0))
+    assert torch.equal(out[:kept.numel()], ids[order])
+    assert (out[kept.numel():] == -1).all(), "wrote past the kept pairs"
+
+
 @pytest.mark.parametrize("W,H,tile", [(640, 480, 8), (1920, 1080, 16), (2048, 2048, 8)])
 def test_more_tiles_bit_exact(dev, W, H, tile):
     """4800, 8160 and 65536 tiles: past 4096 tiles the lists come from the
