@@ -1420,9 +1420,13 @@ inline CsPlan cs_plan(int64_t n, int64_t max_chunks = kCsMaxChunks) {
     return {64, ceil_div(n, (int64_t)kCsThreads * 64)};
 }
 
-// Per-chunk counts, the tiles' totals, and the depth sort's tile order.
+// Per-chunk counts, the tiles' totals, and the depth sort's tile order. Rows
+// for the most chunks that any n' <= n plans, not for n's plan alone (whose
+// chunks are longer past each limit), so that scratch for n serves fewer pairs.
 inline int64_t tile_sort_ws_bytes(int64_t n, int nb, int64_t max_chunks = kCsMaxChunks) {
-    return align256(4 * (int64_t)nb * cs_plan(n, max_chunks).nchunks) +
+    const int64_t rows = std::max(cs_plan(n, max_chunks).nchunks,
+                                  std::min(max_chunks, ceil_div(n, (int64_t)kCsThreads * 8)));
+    return align256(4 * (int64_t)nb * rows) +
            2 * align256(4 * (int64_t)nb);
 }
 

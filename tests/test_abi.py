@@ -145,3 +145,18 @@ def test_missing_library_raises_instead_of_falling_back(tmp_path, monkeypatch, m
     monkeypatch.setattr(_lib, "_lib", None)
     with pytest.raises(RuntimeError, match="Refusing to silently substitute"):
         _lib.open_library()
+
+
+@pytest.mark.parametrize("query", ["tiles", "lists", "capped"])
+def test_sort_scratch_for_more_pairs_serves_fewer(query):
+    """Around every length at which the tile sort's chunks get longer."""
+    from metal_gauss_amd import _lib
+
+    lib = _lib.open_library()
+    size = {"tiles": lambda n: lib.mg_sort_pairs_by_tile_workspace_bytes(n, 2500),
+            "lists": lib.mg_bin_lists_finish_workspace_bytes,
+            "capped": lambda n: lib.mg_bin_lists_capped_workspace_bytes(1000, n)}[query]
+    ns = sorted({256 * per * chunks + d for per in (8, 24, 48, 64)
+                 for chunks in (1, 512, 768, 1024, 1280) for d in (-1, 0, 1)})
+    sizes = [size(n) for n in ns]
+    assert sizes == sorted(sizes)
