@@ -38,6 +38,7 @@
 //   across MI355X's eight XCD L2s). There is one set per (Gaussian, tile)
 //   rather than per (Gaussian, wave).
 #include "mg_common.h"
+#include "raster_slots.h"
 
 namespace mg {
 
@@ -181,7 +182,7 @@ struct Stage {
 };
 static_assert(kBatch <= 256, "list entries are bytes");
 
-constexpr int kGradSlots = 10;   // colour 3, moments 5, sum dg, |d uv|
+constexpr int kGradSlots = grad_rows(true);
 
 // Wave sums of ten values by lane swaps. v_permlane32_swap a, b swaps lanes
 // 32-63 of a with lanes 0-31 of b, leaving (a[0:32], b[0:32]) in a and
@@ -244,11 +245,6 @@ __device__ __forceinline__ void reduce10_to_rows(const float v[10], float &q0, f
 // and the other lanes with bit 1 set hold the zero padding. reduce18_slot
 // names each lane's value, -1 for lanes that deposit nothing. 44 VALU
 // operations for eighteen sums, against 2 x 26 plus twice the deposits.
-__device__ __forceinline__ int reduce18_slot(int lane) {
-    if (lane & 1) return -1;
-    if (lane & 2) return (lane & 0x1C) == 0 ? 8 : -1;
-    return 4 * ((lane >> 2) & 1) + 2 * ((lane >> 3) & 1) + ((lane >> 4) & 1);
-}
 __device__ __forceinline__ float reduce18(const float a[9], const float b[9], int lane) {
     float x0 = a[0], x1 = a[1], x2 = a[2], x3 = a[3], x4 = a[4], x5 = a[5], x6 = a[6];
     float x7 = a[7], x8 = a[8];
@@ -708,7 +704,7 @@ template <int MAXW, bool ABS, bool PIPE>
 __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs A,
                                                                const RasterGrads G,
                                                                const ChunkPlan P) {
-    constexpr int kSlots = ABS ? 10 : 9;
+    constexpr int kSlots = grad_rows(ABS);
     __shared__ StageBwd<MAXW, kSlots> S;
     // Without a plan a workgroup takes a whole tile; with one, one chunk.
     int tile_id, chunk = 0, tile_start, tile_end;
@@ -848,15 +844,9 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
         reduce10_to_rows(v, q0, q1, q2);
         if ((lane & 15) == 0) {
             const int row = lane >> 4;
-            // Row r of q0 holds slot {0,2,1,3}[r], of q1 {4,6,5,7}[r], of
-            // q2 {8,0,9,0}[r]: rows 1 and 3 of q2 are sums of zeros and add
-            // nothing, so all four lanes deposit it (to slots 8, 8, 9, 9; a
-            // lane-dependent address, which the compiler does not turn into
-            // a wave-aggregation loop as it does a single lane's).
-            const int s0 = (row & 1) * 2 + (row >> 1);
-            atomicAdd(&S.grad[s0][j], q0);
-            atomicAdd(&S.grad[4 + s0][j], q1);
-            atomicAdd(&S.grad[8 + (row >> 1)][j], q2);
+            atomicAdd(&S.grad[deposit_row(0, row, ABS)][j], q0);
+            atomicAdd(&S.grad[deposit_row(1, row, ABS)][j], q1);
+            atomicAdd(&S.grad[deposit_row(2, row, ABS)][j], q2);
         }
     };
 
