@@ -17,6 +17,7 @@
 //   * the threshold is 2 * log(255 op) taken in double and rounded once to
 //     fp32, i.e. the correctly rounded value, rather than a fast fp32 log
 //     whose last bit differs between libraries.
+#include "bin_words.h"
 #include "mg_common.h"
 #include "mg_sort.h"
 
@@ -416,31 +417,6 @@ __device__ __forceinline__ void strip_walk(const BinRec &r, const StripPlan &P, 
     // The slice is rewritten for the wave's next rectangle.
     __builtin_amdgcn_wave_barrier();
 }
-
-// The count pass keeps each large rectangle's claims, one 64-bit word per
-// walk step (the wave's ballot of that step's claims), so the write pass
-// replays the steps instead of testing every tile again. A count workgroup
-// has kBlockWords words, taken by its rectangles as their walks start; a
-// rectangle whose steps no longer fit is walked again by the write pass.
-// Its mask word records where its words are: 1 + the first word's index, the
-// step count from bit kWordSteps and the walk's rows a step, less one, from
-// bit kWordRows (0: not kept).
-constexpr int kBlockWords = 1024;
-constexpr int kWordSteps = 11, kWordRows = 22;
-static_assert(kBlockWords < (1 << kWordSteps), "the first word's index + 1 fits below the steps");
-static_assert(kBlockWords < (1 << (kWordRows - kWordSteps)), "the steps fit below the rows");
-
-__device__ __forceinline__ uint32_t kept_mask(int first, int nst, int R) {
-    return (uint32_t)(first + 1) | ((uint32_t)nst << kWordSteps) |
-           ((uint32_t)(R - 1) << kWordRows);
-}
-__device__ __forceinline__ int kept_first(uint32_t m) {
-    return (int)(m & ((1u << kWordSteps) - 1u)) - 1;
-}
-__device__ __forceinline__ int kept_steps(uint32_t m) {
-    return (int)(m >> kWordSteps & ((1u << (kWordRows - kWordSteps)) - 1u));
-}
-__device__ __forceinline__ int kept_rows(uint32_t m) { return (int)(m >> kWordRows) + 1; }
 
 __device__ __forceinline__ int rec_area(const BinRec &r) {
     return ((int)(r.xs >> 16) - (int)(r.xs & 0xffffu) + 1) *
@@ -1135,13 +1111,12 @@ __global__ __launch_bounds__(kBinThreads) void bin_write_rec_kernel(
     int small_cap = 0;        // pairs this thread stages (0 unless a small rectangle)
     int32_t g = 0;
     BinRec r{};
-    uint32_t mask = 0;
     const int cap = k < N ? counts[k] : 0;
+    const uint32_t mask = k < N ? masks[k] : 0u;
     {
-        if (cap > 0) {
+        if (write_takes(cap, mask)) {
             g = (int32_t)k;
             r = recs[g];
-            mask = masks[g];
             if (rec_area(r) > kMaskArea) {
                 big = true;
                 s_rec[tid] = r;
@@ -1216,7 +1191,8 @@ __global__ __launch_bounds__(kBinThreads) void bin_write_rec_kernel(
         for (int q = 0; q < 4; ++q) {
             const int i = i0 + q;
             if (i >= wext) break;
-            const int st = max(hp[q], ex_m) - 1;      // the run's first word
+            // The run's first word: word 0 starts one (see write_takes).
+            const int st = max(hp[q], ex_m) - 1;
             const int j = (int)s_hown[st] - 1;
             const int t = i - st, nr = s_pnr[j];
             const int kk = small_div(t, nr), u = t - kk * nr;

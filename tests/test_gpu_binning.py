@@ -252,6 +252,66 @@ def test_rectangles_of_every_mask_size_bit_exact(dev, shape, ellipse):
     assert np.array_equal(gids.cpu().numpy(), rids), "gauss_ids differ"
 
 
+@pytest.mark.parametrize("kind", ["words", "walks", "both", "all"])
+def test_blocks_whose_first_kept_words_claim_nothing_bit_exact(dev, kind):
+    """Rectangles that keep words and claim no tile: the box meets the image,
+    the ellipse, far outside it, does not. In the first block all rectangles of
+    33 to 64 tiles (whose words come first), or most of the walked ones, or
+    both are such, in the second ("all": in the first too) every large one;
+    the third has none. Exactly the oracle's lists."""
+    from metal_gauss_amd.backend import _bin
+
+    rng = np.random.default_rng(79)
+    N, W, H, tile = 768, 640, 480, 16
+    f32 = np.float32
+    uv = np.stack([rng.uniform(0, W, N), rng.uniform(0, H, N)], 1)
+    rxy = rng.uniform(5, 120, (N, 2))
+    sig = rxy / 3.0
+    idle = np.zeros(N, bool)
+    idle[256:512:3] = True
+    idle[1:256:2] = True
+    idle[[0, 128]] = True
+    at = np.flatnonzero(idle)
+    # A box of w x h tiles at the image's left edge, its Gaussian 400 pixels off.
+    wide = {"words": np.zeros(at.size, bool), "walks": np.ones(at.size, bool),
+            "both": at % 4 == 0, "all": at % 4 == 0}[kind]
+    w = np.where(wide, rng.integers(8, 30, at.size), rng.integers(4, 8, at.size))
+    h = np.where(wide, rng.integers(9, 25, at.size), 9)
+    uv[at, 0] = -400.0
+    rxy[at, 0] = 400.0 + 16 * w - 8
+    rxy[at, 1] = 8 * h - 4
+    uv[at, 1] = 16 * rng.integers(0, H // 16 - h + 1) + 8 * h
+    sig[at] = 4.0
+    if kind == "all":
+        small = np.setdiff1d(np.arange(512), at)
+        rxy[small], sig[small] = 20.0, 7.0
+    elif kind == "words":
+        # Nothing else of the first block lies between 33 and 64 tiles.
+        own = np.setdiff1d(np.arange(256), at)
+        rxy[own] = np.where(own[:, None] % 8 == 2, 100.0, 30.0)
+        uv[own] = rng.uniform(200, 280, (own.size, 2))
+        sig[own] = rxy[own] / 3.0
+    a, c = 1 / sig[:, 0] ** 2, 1 / sig[:, 1] ** 2
+    conic = np.stack([a, np.zeros(N), c], 1).astype(f32)
+    uv, rxy = uv.astype(f32), rxy.astype(f32)
+    op = rng.uniform(0.05, 0.99, N).astype(f32)
+    valid = np.ones(N, np.int32)
+    depth = rng.uniform(0.5, 20.0, N).astype(f32)
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(dev)
+    gids, offs, _ = _bin(t(uv), t(rxy), t(depth), t(valid), t(conic), t(op), W, H, tile)
+    rids, roffs, _, _ = binning_ref.build_tile_lists(uv, rxy, conic, op, valid, depth, W, H,
+                                                     tile, ellipse=True)
+    claims = np.bincount(rids, minlength=N)
+    boxes = np.bincount(binning_ref.build_tile_lists(uv, rxy, conic, op, valid, depth, W, H,
+                                                     tile, ellipse=False)[0], minlength=N)
+    assert not claims[idle].any() and (boxes[idle] > 32).all() and claims[512:].all()
+    if kind == "words":
+        assert (boxes[:256][~idle[:256]] <= 32).any() and (boxes[:256][~idle[:256]] > 64).any()
+        assert not ((boxes[:256] > 32) & (boxes[:256] <= 64) & ~idle[:256]).any()
+    assert np.array_equal(offs.cpu().numpy(), roffs), "tile offsets differ"
+    assert np.array_equal(gids.cpu().numpy(), rids), "gauss_ids differ"
+
+
 @pytest.mark.parametrize("ellipse", [True, False])
 def test_kept_and_rewalked_large_rectangles_bit_exact(dev, ellipse):
     """The count pass keeps a large rectangle's claims as one 64-bit word per

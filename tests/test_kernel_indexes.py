@@ -69,3 +69,63 @@ def test_a_row_past_the_sums_does_not_build(tmp_path):
     """Nine rows with the deposits of ten."""
     with pytest.raises(RuntimeError, match="every deposit has its row"):
         _run(tmp_path, "raster_slots.h", "", edit=(": 8 - (r >> 1)", ": 8 + (r >> 1)"))
+
+
+# One block of the binning's passes, reduced to its bookkeeping: rectangle t
+# has the words steps[t] (0: a small rectangle or none) and claims[t] tiles. The
+# count pass gives the words out in order while they fit; the write pass marks
+# the run starts of the rectangles it takes up, and each word up to the last
+# marked run's end belongs to the last start at or before it.
+REPLAY = """
+    const int steps[] = {%s}, claims[] = {%s};
+    const int n = sizeof steps / sizeof steps[0];
+    int used = 0, ext = 0, owner[kBlockWords] = {}, mark[kBlockWords] = {};
+    for (int t = 0; t < n; ++t) {
+        uint32_t mask = 0;
+        if (steps[t] > 0) {
+            if (used + steps[t] <= kBlockWords) {
+                mask = kept_mask(used, steps[t], 1 + t %% 64);
+                if (kept_rows(mask) != 1 + t %% 64 || kept_steps(mask) != steps[t]) return 1;
+                for (int i = 0; i < steps[t]; ++i) owner[used + i] = t + 1;
+            }
+            used += steps[t] < kBlockWords + 1 ? steps[t] : kBlockWords + 1;
+        } else {
+            mask = claims[t] > 0;
+        }
+        if (write_takes(claims[t], mask) && steps[t] > 0 && mask != 0) {
+            mark[kept_first(mask)] = t + 1;
+            const int end = kept_first(mask) + kept_steps(mask);
+            if (end > ext) ext = end;
+        }
+    }
+    for (int i = 0, st = -1; i < ext; ++i) {
+        if (mark[i]) st = i;
+        std::printf("%%d %%d\\n", owner[i], st < 0 ? -1 : mark[st]);
+    }"""
+
+BLOCKS = {
+    "first claims nothing": ([3, 5, 1, 0], [0, 40, 7, 9]),
+    "one word, nothing": ([1, 1, 1], [0, 0, 2]),
+    "one in the middle": ([2, 700, 4], [9, 0, 3]),
+    "none claims": ([0, 6, 1], [0, 0, 0]),
+    "last does not fit": ([1, 1020, 900, 3], [0, 0, 500, 5]),
+    "words to the last": ([1, 1022, 1], [0, 12, 3]),
+}
+
+
+@pytest.mark.parametrize("block", list(BLOCKS))
+def test_every_kept_word_lies_in_its_rectangles_run(tmp_path, block):
+    steps, claims = BLOCKS[block]
+    rows = _run(tmp_path, "bin_words.h",
+                REPLAY % (", ".join(map(str, steps)), ", ".join(map(str, claims))))
+    assert rows
+    assert all(run == own for own, run in rows), "a word in no run, or in another's"
+
+
+def test_unmarked_runs_without_claims_would_be_found(tmp_path):
+    """Taking up only the rectangles that claim tiles leaves words in no run."""
+    steps, claims = BLOCKS["first claims nothing"]
+    rows = _run(tmp_path, "bin_words.h",
+                REPLAY % (", ".join(map(str, steps)), ", ".join(map(str, claims))),
+                edit=("return count > 0 || mask != 0u;", "return count > 0;"))
+    assert [-1, -1, -1] == [run for own, run in rows if own == 1]
