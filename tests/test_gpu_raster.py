@@ -112,8 +112,8 @@ def test_forward_matches_contract(dev, tile, t_min):
 
 @pytest.mark.parametrize("t_min", [0.3, 1.0, 2.0])
 def test_forward_stops_at_large_thresholds(dev, t_min):
-    """From a threshold of 1 up a pixel holds its first splat alone; the
-    coverage is 1 - T. Bars as above."""
+    """From a threshold of 1 up a pixel holds its first splat alone. Bars as
+    above."""
     W, H, tile = 100, 63, 16
     args = prepare(600, 17, W, H, tile, dev)
     rgb, alpha, T, stop, _ = gpu_forward(args, W, H, tile, t_min)
@@ -122,8 +122,33 @@ def test_forward_stops_at_large_thresholds(dev, t_min):
     assert np.abs(np_(rgb) - r[0])[ok].max() < 1e-4
     assert np.abs(np_(alpha) - r[1])[ok].max() < 1e-4
     assert (np_(stop) == r[3])[ok].all(), "stop indices differ"
-    # 1 - T is rounded once from T, which lies in [0, 1].
-    assert np.array_equal(np_(alpha), np.float32(1.0) - np_(T))
+
+
+@pytest.mark.parametrize("n,t_min", [(40, 1e-4), (600, 1e-4), (600, 2.0)])
+def test_coverage_keeps_the_bits_of_faint_pixels(dev, n, t_min):
+    """Splats whose red is 1 sum their weights in red too. A coverage below
+    0.02 is that of at most five splats (each at least 0.98 / 255), whose two
+    sums are within six roundings of 2^-24 each of the same value; 1 - T would
+    be off by up to 2^-25, 8e-6 of a splat of 1/255. With t_min above 1 a pixel
+    has one splat and the coverage is its alpha, exactly. From T = 0.4 down the
+    coverage is 1 - T."""
+    W, H, tile = 100, 63, 16
+    uv, conic, op, col, gids, offs, tx = prepare(n, 23, W, H, tile, dev)
+    op = op * 0.02 + 0.004     # faint: alphas from 1/255 to 0.021
+    op[::3] = 0.9 if n > 40 else 0.3
+    args = (uv, conic, op, torch.ones_like(col), gids, offs, tx)
+    rgb, alpha, T, stop, _ = gpu_forward(args, W, H, tile, t_min)
+    red, cov, t = (np_(x).astype(np.float64) for x in (rgb[..., 0], alpha, T))
+    faint = (red > 0) & (red < 0.02)
+    off = np.abs(cov - red)[faint] / red[faint]
+    assert faint.sum() > 50 and off.max() <= 2 * 6 * 2.0 ** -24
+    # The other expression would not pass.
+    assert (np.abs(1.0 - t - red)[faint] / red[faint]).max() > 2 * 6 * 2.0 ** -24
+    opaque = np_(T) < np.float32(0.4)
+    assert opaque.any() or n == 40
+    assert np.array_equal(np_(alpha)[opaque], np.float32(1.0) - np_(T)[opaque])
+    if t_min > 1.0:
+        assert np.array_equal(cov[~opaque], red[~opaque])
 
 
 @pytest.mark.parametrize("chunked", [True, False])
