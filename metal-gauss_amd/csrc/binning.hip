@@ -1369,6 +1369,7 @@ inline int tile_bits(int n_tiles) {
 // offsets. Pairs with a tile >= n_tiles are dropped.
 constexpr int kCsBuckets = 4096;
 constexpr int kCsThreads = 256, kCsWaves = kCsThreads / 64;
+constexpr int kCsMaxPer = 48;           // pairs per lane at most
 constexpr int64_t kCsMaxChunks = 768;   // three workgroups per CU
 // Capacity-bounded lists plan for the capacity, which runs above the pairs
 // actually sorted (by the caller's headroom, or more). At the default
@@ -1383,17 +1384,20 @@ struct CsPlan {
     int64_t nchunks;
 };
 
-// The smallest chunk that needs no more than max_chunks workgroups. 24 pairs a
-// lane keep three workgroups on a CU; 16 and 32 were worse wherever they lay
-// next to it (3.6M pairs over 4056 tiles: 48 us with 16, 40 with 24; 5.1M over
-// 2500: 75 with 32, whose registers leave two workgroups a CU, 59 with 24).
+// The smallest chunk that needs no more than max_chunks workgroups, the
+// longest for any more. 24 pairs a lane keep three workgroups on a CU, 48 two;
+// 16 and 32 were worse wherever they lay next to 24 (3.6M pairs over 4056
+// tiles: 48 us with 16, 40 with 24; 5.1M over 2500: 75 with 32, whose
+// registers leave two workgroups a CU, 59 with 24). 64, whose registers leave
+// one, was worse than 48 in any number of chunks (9.5M {id, depth} pairs over
+// 2500 tiles 234 us, 122 with 48; 40M 793, 455).
 inline CsPlan cs_plan(int64_t n, int64_t max_chunks = kCsMaxChunks) {
-    static const int kPers[] = {8, 24, 48, 64};
+    static const int kPers[] = {8, 24, kCsMaxPer};
     for (int p : kPers) {
         const int64_t nc = ceil_div(n, (int64_t)kCsThreads * p);
-        if (nc <= max_chunks || p == 64) return {p, nc};
+        if (nc <= max_chunks) return {p, nc};
     }
-    return {64, ceil_div(n, (int64_t)kCsThreads * 64)};
+    return {kCsMaxPer, ceil_div(n, (int64_t)kCsThreads * kCsMaxPer)};
 }
 
 // Per-chunk counts, the tiles' totals, and the depth sort's tile order. Rows
@@ -1484,11 +1488,11 @@ __global__ __launch_bounds__(kCsThreads) void count_hist_kernel(const CsPass<V> 
 // sixteenth of the chunks (coalesced rows), the waves' sums are joined
 // through LDS, and each wave writes its running exclusive prefixes. Up to
 // kColRows rows per wave (1024 chunks) all of a wave's rows are requested at
-// once and parked in LDS as 16-bit counts (a chunk holds at most 16384
+// once and parked in LDS as 16-bit counts (a chunk holds at most 12288
 // pairs) for the prefix pass; walking the rows in batches instead makes a
 // chain of dependent HBM round trips (12 us at config 4).
 constexpr int kColRows = 64;
-static_assert((int64_t)kCsThreads * 64 <= 65535, "per-chunk tile counts must fit 16 bits");
+static_assert((int64_t)kCsThreads * kCsMaxPer < 0xFFFF, "per-chunk counts and slots fit 16 bits");
 
 template <typename V>
 __global__ __launch_bounds__(64 * kColWaves) void count_colscan_kernel(const CsPass<V> P,
@@ -1744,7 +1748,7 @@ __global__ __launch_bounds__(kCsThreads) void count_scatter_kernel(const CsPass<
         v[r] = i < left ? (P.ids + pb)[i] : V{};
     }
     uint64_t next = peers_of(t[0]);
-    // Two local slots a word (0xFFFF: none; a chunk's are below 2^14 + 1); t
+    // Two local slots a word (0xFFFF: none; a chunk's are lower); t
     // becomes the slot in the output.
     uint32_t lp[kPer / 2];
 #pragma unroll
@@ -1848,7 +1852,6 @@ static int32_t tile_count_sort(const uint32_t *tiles, const V *ids, int64_t n, i
         MG_CS(8)
         MG_CS(24)
         MG_CS(48)
-        MG_CS(64)
         default: MG_REQUIRE(false, "tile sort: %d pairs per lane", plan.per);
     }
 #undef MG_CS

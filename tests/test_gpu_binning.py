@@ -624,11 +624,12 @@ def test_radix_sort_is_stable_and_exact(dev, n, bits):
 @pytest.mark.parametrize("n,n_tiles,kind", [
     (1, 1, "uniform"), (7, 3, "uniform"), (2049, 300, "uniform"), (300_001, 2500, "uniform"),
     (300_001, 4096, "descending"), (1_000_003, 1, "uniform"), (2_000_000, 2500, "one_hot"),
-    (5_000_011, 2500, "uniform"), (7_000_001, 4096, "uniform"), (100_000, 2500, "dropped")])
+    (5_000_011, 2500, "uniform"), (7_000_001, 4096, "uniform"), (100_000, 2500, "dropped"),
+    (9_500_003, 2501, "dropped"), (9_500_003, 4096, "one_hot")])
 def test_sort_pairs_by_tile_is_stable_and_exact(dev, n, n_tiles, kind):
     """The one-pass counting sort behind mg_bin_lists_finish against numpy's
-    stable argsort: chunk plans from 8 to 64 pairs per lane (n up to 7M),
-    one tile, every pair in one tile, reversed input, and tiles past n_tiles
+    stable argsort: every chunk plan (from 9.4M pairs on its longest chunks in
+    any number), one tile, every pair in one tile, reversed input, and tiles past n_tiles
     (dropped; the last offset counts the rest)."""
     from metal_gauss_amd import _lib
 
@@ -662,12 +663,15 @@ def test_sort_pairs_by_tile_is_stable_and_exact(dev, n, n_tiles, kind):
 
 
 @pytest.mark.parametrize("n_tiles", [1, 2, 63, 255, 257, 2501, 4095, 4096])
-@pytest.mark.parametrize("n", [2047, 2048, 2049, 1_600_000, 1_578_241, 4_800_003])
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 1_600_000, 1_578_241, 4_718_593, 4_800_003,
+                               9_437_184, 9_437_185, 12_582_912, 12_582_913])
 def test_sort_pairs_by_tile_at_the_edges_of_its_windows(dev, n, n_tiles):
     """Chunks of 2048, 6144 and 12288 pairs leave through LDS windows of 2048
     or 3072; the last chunk holds one pair, a whole window, or part of one, and
     a tenth of the pairs is dropped, so windows end anywhere. Even and odd
-    tile counts (the counters are two to a word), up to the most."""
+    tile counts (the counters are two to a word), up to the most. 768 of the
+    longest chunks and one pair more, and as many chunks as the column scan
+    holds at once (1024) and one more."""
     from metal_gauss_amd import _lib
 
     lib = _lib.load()

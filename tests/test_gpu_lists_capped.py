@@ -91,6 +91,55 @@ def test_capped_lists_equal_the_two_call_lists(dev, case, cap):
         assert (got_offs == 0).all(), "an overflowed build must leave every list empty"
 
 
+@pytest.mark.parametrize("capped", [False, True])
+@pytest.mark.parametrize("n,headroom", [(3780, 1.0), (3780, 1.7), (5040, 1.25), (5240, 1.01)])
+def test_lists_of_many_million_pairs(dev, n, headroom, capped):
+    """Rectangles over all 2500 tiles, or over the left half of them: 9.4 to
+    13.1M {id, depth} pairs, on both sides of the tile sort's longest chunks'
+    first limit, of its limit for a capacity and of 1024 chunks. A tile's list
+    is the Gaussians that cover it in depth order, ties in order of id."""
+    from metal_gauss_amd import _lib, backend
+
+    W = H = 800
+    g = np.random.default_rng(n)
+    half = np.zeros(n, bool)
+    half[g.integers(0, n, 24)] = True
+    uv = np.full((n, 2), 400.0, np.float32)
+    uv[half, 0] = 200.0
+    rxy = np.full((n, 2), 399.0, np.float32)
+    rxy[half, 0] = 199.0
+    depth = np.round(g.uniform(1.0, 30.0, n) * 64).astype(np.float32) / 64
+    t = lambda x: torch.from_numpy(x).to(dev)
+    args = (t(uv), t(rxy), t(depth), torch.ones(n, dtype=torch.int32, device=dev), None, None, W,
+            H, 16)
+    order = np.argsort(depth, kind="stable")
+    total = n * 2500 - int(half.sum()) * 1250
+    if capped:
+        lib = _lib.load()
+        cap = int(total * headroom)
+        ids = torch.full((cap,), -7, dtype=torch.int32, device=dev)
+        offs = torch.full((2501,), -7, dtype=torch.int32, device=dev)
+        status = torch.full((2,), -7, dtype=torch.int64, device=dev)
+        ws = torch.empty(lib.mg_bin_lists_capped_workspace_bytes(n, cap), dtype=torch.uint8,
+                         device=dev)
+        _lib.check(lib.mg_bin_lists_capped(
+            n, args[0].data_ptr(), args[1].data_ptr(), None, None, args[3].data_ptr(),
+            args[2].data_ptr(), W, H, 16, 50, 50, cap, ids.data_ptr(), offs.data_ptr(),
+            status.data_ptr(), None, 0, ws.data_ptr(), ws.numel(), None, _lib.stream(ids)))
+        assert status.tolist() == [total, 0]
+    else:
+        ids, offs, _ = backend._bin(*args)
+        assert ids.numel() == total
+    offs = offs.cpu().numpy()
+    tiles = np.arange(2500) % 50 < 25
+    lens = np.where(tiles, n, n - int(half.sum()))
+    assert offs[0] == 0 and np.array_equal(np.diff(offs), lens)
+    left = torch.from_numpy(order.astype(np.int32)).to(dev)
+    right = torch.from_numpy(order[~half[order]].astype(np.int32)).to(dev)
+    rows = torch.cat([left.repeat(25), right.repeat(25)]).repeat(50)
+    assert torch.equal(ids[:total], rows)
+
+
 def _mip_projection(s, dev, tile):
     """The mip projection with its per-block binning work estimate:
     (uv, conic, depth, rxy, valid, opacity_eff), block_work."""
