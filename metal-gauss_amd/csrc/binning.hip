@@ -1369,14 +1369,14 @@ inline int tile_bits(int n_tiles) {
 // offsets. Pairs with a tile >= n_tiles are dropped.
 constexpr int kCsBuckets = 4096;
 constexpr int kCsThreads = 256, kCsWaves = kCsThreads / 64;
-constexpr int kCsMaxPer = 48;           // pairs per lane at most
 constexpr int64_t kCsMaxChunks = 768;   // three workgroups per CU
 // Capacity-bounded lists plan for the capacity, which runs above the pairs
-// actually sorted (by the caller's headroom, or more). At the default
-// headroom of a quarter the kept pairs of a full plan are 1024 chunks, what
-// the column scan holds at once; with the exact limit a headroom that crossed
-// it would lengthen the chunks a step and leave part of the GPU idle.
-constexpr int64_t kCsMaxChunksCapped = 1280;
+// actually sorted (by the caller's headroom, or more); with the exact limit a
+// headroom that crossed it would lengthen the chunks a step and leave part of
+// the GPU idle. At the default headroom of a quarter the kept pairs of a full
+// plan are the exact limit's.
+constexpr int64_t kCsMaxChunksCapped = 960;
+constexpr int64_t kCsMaxLong = 512;     // two workgroups per CU
 constexpr int kColWaves = 16;           // waves of the column scan's workgroups
 
 struct CsPlan {
@@ -1384,28 +1384,32 @@ struct CsPlan {
     int64_t nchunks;
 };
 
-// The smallest chunk that needs no more than max_chunks workgroups, the
-// longest for any more. 24 pairs a lane keep three workgroups on a CU, 48 two;
-// 16 and 32 were worse wherever they lay next to 24 (3.6M pairs over 4056
-// tiles: 48 us with 16, 40 with 24; 5.1M over 2500: 75 with 32, whose
-// registers leave two workgroups a CU, 59 with 24). 64, whose registers leave
-// one, was worse than 48 in any number of chunks (9.5M {id, depth} pairs over
-// 2500 tiles 234 us, 122 with 48; 40M 793, 455).
-inline CsPlan cs_plan(int64_t n, int64_t max_chunks = kCsMaxChunks) {
-    static const int kPers[] = {8, 24, kCsMaxPer};
-    for (int p : kPers) {
-        const int64_t nc = ceil_div(n, (int64_t)kCsThreads * p);
-        if (nc <= max_chunks) return {p, nc};
-    }
-    return {kCsMaxPer, ceil_div(n, (int64_t)kCsThreads * kCsMaxPer)};
+// The smallest chunk that needs no more workgroups than the limit, else 24
+// pairs a lane in any number of chunks; but between 768 chunks of 24 and 512 of
+// 48 (exact counts), where those of 24 would start a fourth workgroup a CU on
+// their own, 48, which leave two. {id, depth} pairs over 2500 tiles took, with
+// 8 / 16 / 24 / 48 a lane: 1.8M pairs 41 / 37 / 42 / 58 us, 2.5M 51 / 41 / 43 /
+// 59, 3.5M 70 / 50 / 49 / 67, 4.8M 91 / 68 / 71 / 69, 6.5M 115 / 88 / 83 / 110,
+// 9.5M 157 / 118 / 116 / 123, 20M 357 / 271 / 224 / 251; over 256 tiles 24 is a
+// sixth faster than 48 from 9.5M on, over 4096 as fast. 32 and 64, whose
+// registers leave two workgroups and one, lay above 24 in any number of chunks
+// (9.5M: 133 and 234).
+inline CsPlan cs_plan(int64_t n, bool capped) {
+    auto chunks = [n](int per) { return ceil_div(n, (int64_t)kCsThreads * per); };
+    const int64_t limit = capped ? kCsMaxChunksCapped : kCsMaxChunks;
+    for (int p : {8, 16})
+        if (chunks(p) <= limit) return {p, chunks(p)};
+    if (!capped && chunks(24) > limit && chunks(48) <= kCsMaxLong) return {48, chunks(48)};
+    return {24, chunks(24)};
 }
 
 // Per-chunk counts, the tiles' totals, and the depth sort's tile order. Rows
 // for the most chunks that any n' <= n plans, not for n's plan alone (whose
 // chunks are longer past each limit), so that scratch for n serves fewer pairs.
-inline int64_t tile_sort_ws_bytes(int64_t n, int nb, int64_t max_chunks = kCsMaxChunks) {
-    const int64_t rows = std::max(cs_plan(n, max_chunks).nchunks,
-                                  std::min(max_chunks, ceil_div(n, (int64_t)kCsThreads * 8)));
+inline int64_t tile_sort_ws_bytes(int64_t n, int nb, bool capped = false) {
+    const int64_t limit = capped ? kCsMaxChunksCapped : kCsMaxChunks;
+    const int64_t rows = std::max(cs_plan(n, capped).nchunks,
+                                  std::min(limit, ceil_div(n, (int64_t)kCsThreads * 8)));
     return align256(4 * (int64_t)nb * rows) +
            2 * align256(4 * (int64_t)nb);
 }
@@ -1492,7 +1496,7 @@ __global__ __launch_bounds__(kCsThreads) void count_hist_kernel(const CsPass<V> 
 // pairs) for the prefix pass; walking the rows in batches instead makes a
 // chain of dependent HBM round trips (12 us at config 4).
 constexpr int kColRows = 64;
-static_assert((int64_t)kCsThreads * kCsMaxPer < 0xFFFF, "per-chunk counts and slots fit 16 bits");
+static_assert((int64_t)kCsThreads * 48 < 0xFFFF, "per-chunk counts and slots fit 16 bits");
 
 template <typename V>
 __global__ __launch_bounds__(64 * kColWaves) void count_colscan_kernel(const CsPass<V> P,
@@ -1812,11 +1816,11 @@ static int32_t tile_count_sort(const uint32_t *tiles, const V *ids, int64_t n, i
                                int32_t **depth_order = nullptr) {
     MG_REQUIRE(n > 0 && n < (1LL << 31) && n_tiles >= 1 && n_tiles <= kCsBuckets,
                "tile sort: %lld pairs over %d tiles", (long long)n, n_tiles);
-    const int64_t max_chunks = status ? kCsMaxChunksCapped : kCsMaxChunks;
-    MG_REQUIRE(ws && ws_bytes >= tile_sort_ws_bytes(n, n_tiles, max_chunks),
+    const bool capped = status != nullptr;
+    MG_REQUIRE(ws && ws_bytes >= tile_sort_ws_bytes(n, n_tiles, capped),
                "tile sort: workspace %lld bytes, need %lld", (long long)ws_bytes,
-               (long long)tile_sort_ws_bytes(n, n_tiles, max_chunks));
-    const CsPlan plan = cs_plan(n, max_chunks);
+               (long long)tile_sort_ws_bytes(n, n_tiles, capped));
+    const CsPlan plan = cs_plan(n, capped);
     CsPass<V> P{};
     P.tiles = tiles;
     P.ids = ids;
@@ -1850,6 +1854,7 @@ static int32_t tile_count_sort(const uint32_t *tiles, const V *ids, int64_t n, i
         break;
     switch (plan.per) {
         MG_CS(8)
+        MG_CS(16)
         MG_CS(24)
         MG_CS(48)
         default: MG_REQUIRE(false, "tile sort: %d pairs per lane", plan.per);
@@ -2417,8 +2422,7 @@ static int32_t check_bin_args(const char *who, int64_t N, const void *uv, const 
 // sort's per-chunk counts at its largest tile count.
 static int64_t finish_sort_bytes(int64_t T, bool capped) {
     return align256(std::max(sort_ws_bytes(T),
-                             tile_sort_ws_bytes(T, kCsBuckets,
-                                                capped ? kCsMaxChunksCapped : kCsMaxChunks)));
+                             tile_sort_ws_bytes(T, kCsBuckets, capped)));
 }
 
 // Pairs in Gaussian order, grouped by tile, then each tile's list sorted by

@@ -628,8 +628,7 @@ def test_radix_sort_is_stable_and_exact(dev, n, bits):
     (9_500_003, 2501, "dropped"), (9_500_003, 4096, "one_hot")])
 def test_sort_pairs_by_tile_is_stable_and_exact(dev, n, n_tiles, kind):
     """The one-pass counting sort behind mg_bin_lists_finish against numpy's
-    stable argsort: every chunk plan (from 9.4M pairs on its longest chunks in
-    any number), one tile, every pair in one tile, reversed input, and tiles past n_tiles
+    stable argsort: every chunk plan, one tile, every pair in one tile, reversed input, and tiles past n_tiles
     (dropped; the last offset counts the rest)."""
     from metal_gauss_amd import _lib
 
@@ -663,15 +662,16 @@ def test_sort_pairs_by_tile_is_stable_and_exact(dev, n, n_tiles, kind):
 
 
 @pytest.mark.parametrize("n_tiles", [1, 2, 63, 255, 257, 2501, 4095, 4096])
-@pytest.mark.parametrize("n", [2047, 2048, 2049, 1_600_000, 1_578_241, 4_718_593, 4_800_003,
-                               9_437_184, 9_437_185, 12_582_912, 12_582_913])
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 1_600_000, 1_578_241, 1_572_864, 1_572_865,
+                               3_145_728, 3_145_729, 4_718_592, 4_718_593, 4_800_003, 6_291_456,
+                               6_291_457, 12_582_913])
 def test_sort_pairs_by_tile_at_the_edges_of_its_windows(dev, n, n_tiles):
-    """Chunks of 2048, 6144 and 12288 pairs leave through LDS windows of 2048
-    or 3072; the last chunk holds one pair, a whole window, or part of one, and
-    a tenth of the pairs is dropped, so windows end anywhere. Even and odd
-    tile counts (the counters are two to a word), up to the most. 768 of the
-    longest chunks and one pair more, and as many chunks as the column scan
-    holds at once (1024) and one more."""
+    """Chunks of 2048, 4096, 6144 and 12288 pairs leave through LDS windows of
+    2048 or 3072; the last chunk holds one pair, a whole window, or part of
+    one, and a tenth of the pairs is dropped, so windows end anywhere. Even and
+    odd tile counts (the counters are two to a word), up to the most. Lengths
+    on both sides of every change of chunk, the last of them also of the 1024
+    chunks that the column scan holds at once, and twice that."""
     from metal_gauss_amd import _lib
 
     lib = _lib.load()

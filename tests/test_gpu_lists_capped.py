@@ -92,12 +92,14 @@ def test_capped_lists_equal_the_two_call_lists(dev, case, cap):
 
 
 @pytest.mark.parametrize("capped", [False, True])
-@pytest.mark.parametrize("n,headroom", [(3780, 1.0), (3780, 1.7), (5040, 1.25), (5240, 1.01)])
+@pytest.mark.parametrize("n,headroom", [(700, 1.1), (700, 1.2), (1440, 1.1), (1440, 1.2),
+                                        (2520, 1.0), (2520, 1.7), (5240, 1.01)])
 def test_lists_of_many_million_pairs(dev, n, headroom, capped):
-    """Rectangles over all 2500 tiles, or over the left half of them: 9.4 to
-    13.1M {id, depth} pairs, on both sides of the tile sort's longest chunks'
-    first limit, of its limit for a capacity and of 1024 chunks. A tile's list
-    is the Gaussians that cover it in depth order, ties in order of id."""
+    """Rectangles over all 2500 tiles, or over the left half of them: 1.7 to
+    13.1M {id, depth} pairs, counts and capacities that take every chunk of the
+    tile sort, the capacities of the first four on both sides of its limits. A
+    tile's list is the Gaussians that cover it in depth order, ties in order of
+    id."""
     from metal_gauss_amd import _lib, backend
 
     W = H = 800
