@@ -125,26 +125,38 @@ __global__ void ssim_chain_bwd_kernel(const float *x, const float *y, const floa
 // in LDS (21.5 instead of 36.3 KB: six workgroups a CU instead of four, 54 ->
 // 50 us for the forward at 1920x1080). Forward and backward: 63 + 46 -> 50 +
 // 34.5 us at 1920x1080, 24.5 + 18.5 -> 20.2 + 16.1 at 800x800.
-constexpr int kTW = 32, kTH = 32;                 // output tile
-constexpr int kIW = kTW + 2 * kR, kIH = kTH + 2 * kR;   // 42 x 42 with halo
+//
+// Up to three workgroups a CU tiles have 16 rows: there a call takes one
+// workgroup's time, which is shorter with half the rows and half the runs
+// (forward + backward 7.8 + 4.7 -> 6.7 + 3.7 us at 128x128, 8.1 + 4.8 -> 7.5 +
+// 4.6 at 256x256, 9.3 + 5.9 -> 9.1 + 5.4 at 300x400; past it 9.4 + 5.9 -> 10.0
+// + 6.0 at 320x480).
+constexpr int kTW = 32;                           // columns of an output tile
+constexpr int kIW = kTW + 2 * kR;                 // 42 with halo
 constexpr int kIWP = 44;                          // LDS row stride: 16-byte rows
 constexpr int kSsimThreads = 256;
-// Register blocking of the separable blur: a horizontal task makes kHRun
-// neighbouring outputs of one row from one read of its kHRun + 2 kR inputs;
-// a vertical task makes kVRun outputs of one column.
-constexpr int kHRun = 8, kVRun = 4;
-constexpr int kHIn = 20;                          // inputs read: five float4s
-constexpr int kHTasks = kIH * (kTW / kHRun);      // 168
-constexpr int kVTasks = (kTH / kVRun) * kTW;      // 256
-static_assert(kHTasks <= kSsimThreads && kVTasks == kSsimThreads, "blur tasks per thread");
-static_assert(kHRun + 2 * kR <= kHIn && (kTW / kHRun - 1) * kHRun + kHIn <= kIWP,
-              "a horizontal task reads five float4s of its row");
-// Halo elements per thread: thread t loads column t % kIW of rows t / kIW + 6 r
-// (252 of the 256 threads), all requested before any of them is stored to LDS
-// (a rolled loop waits for each in turn).
 constexpr int kLoadRows = kSsimThreads / kIW;     // 6
-constexpr int kLoadIters = kIH / kLoadRows;       // 7
-static_assert(kLoadRows * kLoadIters == kIH, "whole rows of loads");
+constexpr int64_t kSsimSmall = 768;               // work items of 32x16 tiles at most
+
+// The split of an output tile of TH rows, 32 or 16.
+template <int TH>
+struct SsimTile {
+    static constexpr int kIH = TH + 2 * kR;       // rows with halo: 42, 26
+    // Register blocking of the separable blur: a horizontal task makes kHRun
+    // neighbouring outputs of one row from one read of its kHRun + 2 kR inputs;
+    // a vertical task makes kVRun outputs of one column.
+    static constexpr int kHRun = TH / 4, kVRun = TH / 8;
+    static constexpr int kHIn = (kHRun + 2 * kR + 3) / 4 * 4;    // inputs read: whole float4s
+    static constexpr int kHTasks = kIH * (kTW / kHRun);          // 168, 208
+    static_assert(kHTasks <= kSsimThreads && (TH / kVRun) * kTW == kSsimThreads,
+                  "blur tasks per thread");
+    static_assert(kHRun % 4 == 0 && (kTW / kHRun - 1) * kHRun + kHIn <= kIWP,
+                  "a horizontal task's float4s lie in its row");
+    // Halo elements per thread: thread t loads column t % kIW of rows t / kIW +
+    // 6 r (252 of the 256 threads), all requested before any of them is stored
+    // to LDS (a rolled loop waits for each in turn).
+    static constexpr int kLoadIters = (kIH + kLoadRows - 1) / kLoadRows;   // 7, 5
+};
 
 // Work items of the fused kernels: (output tile, channel) pairs, item =
 // 3 * tile + channel, tile = ty * tiles_x + tx. The items are dealt to the XCDs
@@ -163,6 +175,7 @@ __device__ __forceinline__ SsimItem ssim_item(int tiles_x) {
 // The horizontal task of thread t: row t / (kTW / kHRun), first output column
 // kHRun * (t % (kTW / kHRun)); its inputs are kHIn floats of that LDS row from
 // the same column.
+template <int kHRun, int kHIn>
 __device__ __forceinline__ void h_inputs(const float (*src)[kIWP], int t, int &row, int &c0,
                                          float (&v)[kHIn]) {
     row = t / (kTW / kHRun);
@@ -199,10 +212,14 @@ __device__ __forceinline__ void ssim_terms(float mx, float my, float edd, float 
 
 // block_sums[b] gets work item b's SSIM sum; with l1_sums, l1_sums[b] gets
 // its sum of |x - y| over the same pixels and channel.
+template <int TH>
 __global__ __launch_bounds__(kSsimThreads) __attribute__((amdgpu_waves_per_eu(6))) void
 ssim_fused_fwd_kernel(
     const float *x, const float *y, const float *__restrict__ w, int H, int W, int tiles_x,
     float *partials, float *block_sums, float *l1_sums) {
+    using Tile = SsimTile<TH>;
+    constexpr int kIH = Tile::kIH, kHRun = Tile::kHRun, kVRun = Tile::kVRun, kHIn = Tile::kHIn;
+    constexpr int kHTasks = Tile::kHTasks, kLoadIters = Tile::kLoadIters;
     // The horizontal pass's maps take the images' place: every task holds its
     // results in registers across a barrier.
     __shared__ __align__(16) union {
@@ -217,7 +234,7 @@ ssim_fused_fwd_kernel(
     __shared__ float s_red[2][kSsimThreads / 64];
     const SsimItem it = ssim_item(tiles_x);
     const int c = it.c;
-    const int x0 = it.tx * kTW - kR, y0 = it.ty * kTH - kR;
+    const int x0 = it.tx * kTW - kR, y0 = it.ty * TH - kR;
     const int tid = threadIdx.x;
     float wk[2 * kR + 1];
 #pragma unroll
@@ -240,6 +257,7 @@ ssim_fused_fwd_kernel(
         if (ly < kLoadRows) {
 #pragma unroll
             for (int r = 0; r < kLoadIters; ++r) {
+                if (kIH % kLoadRows != 0 && ly + kLoadRows * r >= kIH) continue;
                 s_x[ly + kLoadRows * r][lx] = xv[r];
                 s_y[ly + kLoadRows * r][lx] = yv[r];
             }
@@ -261,14 +279,14 @@ ssim_fused_fwd_kernel(
 #pragma unroll
     for (int o = 0; o < kVRun; ++o) {
         const float l1 = fabsf(s_x[r0 + o + kR][lx + kR] - s_y[r0 + o + kR][lx + kR]);
-        local_l1 += gx < W && it.ty * kTH + r0 + o < H ? l1 : 0.f;
+        local_l1 += gx < W && it.ty * TH + r0 + o < H ? l1 : 0.f;
     }
     int row = 0, c0 = 0;
     float m[4][kHRun] = {};
     if (tid < kHTasks) {
         float xv[kHIn], yv[kHIn];
-        h_inputs(s_x, tid, row, c0, xv);
-        h_inputs(s_y, tid, row, c0, yv);
+        h_inputs<kHRun>(s_x, tid, row, c0, xv);
+        h_inputs<kHRun>(s_y, tid, row, c0, yv);
 #pragma unroll
         for (int j = 0; j < kHRun + 2 * kR; ++j) {
             const float a = xv[j], b = yv[j], dd = (a - b) * (a - b), ab = a * b;
@@ -314,7 +332,7 @@ ssim_fused_fwd_kernel(
         }
 #pragma unroll
         for (int o = 0; o < kVRun; ++o) {
-            const int gy = it.ty * kTH + r0 + o;
+            const int gy = it.ty * TH + r0 + o;
             if (gx >= W || gy >= H) continue;
             float S, pm, pxx, pxy;
             ssim_terms(m[o][0], m[o][1], m[o][2], m[o][3], S, pm, pxx, pxy);
@@ -419,10 +437,14 @@ __global__ __launch_bounds__(256) void photometric_loss_kernel(const float *ssim
 // dx = g / (3N) * (a_ssim * dSSIM_sum/dx + a_l1 * sign(x - y)), g = scale_dev[0]:
 // a_ssim = 1, a_l1 = 0 is the gradient of the SSIM mean; a_ssim = -lam,
 // a_l1 = 1 - lam that of the photometric loss.
+template <int TH>
 __global__ __launch_bounds__(kSsimThreads) __attribute__((amdgpu_waves_per_eu(6))) void
 ssim_fused_bwd_kernel(
     const float *x, const float *y, const float *__restrict__ w, const float *partials,
     const float *scale_dev, int H, int W, int tiles_x, float a_ssim, float a_l1, float *dx) {
+    using Tile = SsimTile<TH>;
+    constexpr int kIH = Tile::kIH, kHRun = Tile::kHRun, kVRun = Tile::kVRun, kHIn = Tile::kHIn;
+    constexpr int kHTasks = Tile::kHTasks, kLoadIters = Tile::kLoadIters;
     // As in the forward, the blurred maps take their inputs' place.
     __shared__ __align__(16) union {
         float p[3][kIH][kIWP];
@@ -432,7 +454,7 @@ ssim_fused_bwd_kernel(
     float(*const s_h)[kIH][kTW] = u.h;
     const SsimItem it = ssim_item(tiles_x);
     const int c = it.c;
-    const int x0 = it.tx * kTW - kR, y0 = it.ty * kTH - kR;
+    const int x0 = it.tx * kTW - kR, y0 = it.ty * TH - kR;
     const int tid = threadIdx.x;
     const int64_t N = (int64_t)W * H;
     float wk[2 * kR + 1];
@@ -455,9 +477,11 @@ ssim_fused_bwd_kernel(
         }
         if (ly < kLoadRows) {
 #pragma unroll
-            for (int r = 0; r < kLoadIters; ++r)
+            for (int r = 0; r < kLoadIters; ++r) {
+                if (kIH % kLoadRows != 0 && ly + kLoadRows * r >= kIH) continue;
 #pragma unroll
                 for (int q = 0; q < 3; ++q) s_p[q][ly + kLoadRows * r][lx] = pv[q][r];
+            }
         }
     }
     for (int i = tid; i < kIH * (kIWP - kIW); i += kSsimThreads) {
@@ -472,7 +496,7 @@ ssim_fused_bwd_kernel(
     if (tid < kHTasks) {
         float v[3][kHIn];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) h_inputs(s_p[q], tid, row, c0, v[q]);
+        for (int q = 0; q < 3; ++q) h_inputs<kHRun>(s_p[q], tid, row, c0, v[q]);
 #pragma unroll
         for (int j = 0; j < kHRun + 2 * kR; ++j) {
 #pragma unroll
@@ -514,7 +538,7 @@ ssim_fused_bwd_kernel(
     const int gx = it.tx * kTW + lx;
 #pragma unroll
     for (int o = 0; o < kVRun; ++o) {
-        const int gy = it.ty * kTH + r0 + o;
+        const int gy = it.ty * TH + r0 + o;
         if (gx >= W || gy >= H) continue;
         const int64_t po = ((int64_t)gy * W + gx) * 3 + c;
         const float xv = x[po], yv = y[po];
@@ -528,17 +552,33 @@ ssim_fused_bwd_kernel(
     }
 }
 
-// Work items (workgroups) of the fused kernels: one per (output tile, channel).
+// The block sums a caller's workspace and the static scratch are sized by: one
+// per 32x16 pixels and channel, of which tiles of 32x32 use half.
+inline int64_t ssim_sized_blocks(int H, int W) { return ceil_div(W, kTW) * ceil_div(H, 16) * 3; }
+
+// Rows of an image's output tiles, and its work items (workgroups): one per
+// (output tile, channel).
+inline int ssim_tile_rows(int H, int W) { return ssim_sized_blocks(H, W) <= kSsimSmall ? 16 : 32; }
 inline int64_t ssim_blocks(int H, int W) {
-    return ceil_div(W, kTW) * ceil_div(H, kTH) * 3;
+    return ceil_div(W, kTW) * ceil_div(H, ssim_tile_rows(H, W)) * 3;
 }
 
-// The block sums a caller's workspace and the static scratch are sized by: one
-// per 32x16 pixels and channel, of which the 32x32 tiles use half.
-inline int64_t ssim_sized_blocks(int H, int W) {
-    return ceil_div(W, 32) * ceil_div(H, 16) * 3;
+template <typename... A>
+inline void ssim_fwd_launch(int H, int W, hipStream_t s, A... a) {
+    const unsigned grid = (unsigned)ssim_blocks(H, W);
+    if (ssim_tile_rows(H, W) == 16)
+        ssim_fused_fwd_kernel<16><<<grid, kSsimThreads, 0, s>>>(a...);
+    else
+        ssim_fused_fwd_kernel<32><<<grid, kSsimThreads, 0, s>>>(a...);
 }
-static_assert(kTW >= 32 && kTH >= 16, "no more tiles than sized");
+template <typename... A>
+inline void ssim_bwd_launch(int H, int W, hipStream_t s, A... a) {
+    const unsigned grid = (unsigned)ssim_blocks(H, W);
+    if (ssim_tile_rows(H, W) == 16)
+        ssim_fused_bwd_kernel<16><<<grid, kSsimThreads, 0, s>>>(a...);
+    else
+        ssim_fused_bwd_kernel<32><<<grid, kSsimThreads, 0, s>>>(a...);
+}
 
 // ------------------------------------------------ allocation-free variant
 // mg_photometric_loss_forward_noalloc keeps the loss forward's block sums in
@@ -591,9 +631,8 @@ static int32_t photometric_forward(const float *x, const float *y, const float *
     hipStream_t s = as_stream(stream);
     const int tiles_x = (int)ceil_div(W, kTW);
     const int64_t nb = ssim_blocks(H, W);
-    const unsigned grid = (unsigned)nb;
     TimedScope ts("ssim_fused_forward", s);
-    ssim_fused_fwd_kernel<<<grid, kSsimThreads, 0, s>>>(x, y, w, H, W, tiles_x, partials, sums,
+    ssim_fwd_launch(H, W, s, x, y, w, H, W, tiles_x, partials, sums,
                                                         sums + nb);
     MG_LAUNCHED("ssim_fused_fwd_kernel");
     photometric_loss_kernel<<<1, 256, 0, s>>>(sums, sums + nb, nb, 3LL * H * W, ssim_weight, out);
@@ -677,7 +716,7 @@ int32_t mg_ssim_fused_forward(const float *x, const float *y, const float *w, in
     const unsigned grid = (unsigned)ssim_blocks(H, W);
     float *sums = static_cast<float *>(workspace);
     TimedScope ts("ssim_fused_forward", s);
-    ssim_fused_fwd_kernel<<<grid, kSsimThreads, 0, s>>>(x, y, w, H, W, tiles_x, partials, sums,
+    ssim_fwd_launch(H, W, s, x, y, w, H, W, tiles_x, partials, sums,
                                                         nullptr);
     MG_LAUNCHED("ssim_fused_fwd_kernel");
     ssim_mean_kernel<<<1, 256, 0, s>>>(sums, (int64_t)grid, 3LL * H * W, mean_out);
@@ -692,9 +731,8 @@ int32_t mg_ssim_fused_backward(const float *x, const float *y, const float *w,
                "mg_ssim_fused_backward: bad arguments");
     hipStream_t s = as_stream(stream);
     const int tiles_x = (int)ceil_div(W, kTW);
-    const unsigned grid = (unsigned)ssim_blocks(H, W);
     TimedScope ts("ssim_fused_backward", s);
-    ssim_fused_bwd_kernel<<<grid, kSsimThreads, 0, s>>>(x, y, w, partials, scale_dev, H, W,
+    ssim_bwd_launch(H, W, s, x, y, w, partials, scale_dev, H, W,
                                                         tiles_x, 1.0f, 0.0f, d_x);
     MG_LAUNCHED("ssim_fused_bwd_kernel");
     return MG_OK;
@@ -741,9 +779,8 @@ int32_t mg_photometric_loss_backward(const float *x, const float *y, const float
                (double)ssim_weight);
     hipStream_t s = as_stream(stream);
     const int tiles_x = (int)ceil_div(W, kTW);
-    const unsigned grid = (unsigned)ssim_blocks(H, W);
     TimedScope ts("ssim_fused_backward", s);
-    ssim_fused_bwd_kernel<<<grid, kSsimThreads, 0, s>>>(x, y, w, partials, grad_dev, H, W, tiles_x,
+    ssim_bwd_launch(H, W, s, x, y, w, partials, grad_dev, H, W, tiles_x,
                                                         -ssim_weight, 1.0f - ssim_weight, d_x);
     MG_LAUNCHED("ssim_fused_bwd_kernel");
     return MG_OK;

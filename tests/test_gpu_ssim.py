@@ -117,8 +117,11 @@ def test_photometric_loss_upstream_gradient(dev):
     assert torch.allclose(g2, 2.5 * g1, rtol=1e-5, atol=1e-12)
 
 
-@pytest.mark.parametrize("H,W", [(1, 1), (1, 64), (31, 33), (32, 32), (33, 31), (42, 43), (65, 5)])
+@pytest.mark.parametrize("H,W", [(1, 1), (1, 64), (15, 33), (16, 32), (17, 31), (26, 43), (31, 33),
+                                 (32, 32), (33, 31), (42, 43), (65, 5), (256, 512), (257, 512),
+                                 (266, 491), (289, 481), (288, 483), (33, 8193), (16, 8161)])
 def test_photometric_loss_at_the_edges_of_tiles(dev, H, W):
     """The same expression where an image ends inside, at and just past the
-    kernels' 32x32 tiles and their halo; bars as above."""
+    kernels' tiles (32x16 for up to 768 of them in three channels, 256x512 the
+    last, else 32x32) and their halo; bars as above."""
     test_photometric_loss_matches_the_trainer_expression(dev, H, W, 0.2)
