@@ -71,16 +71,21 @@ __device__ __forceinline__ int64_t sort_count(int64_t n, const int64_t *status) 
     return status ? (status[1] != 0 ? 0 : min(status[0], n)) : n;
 }
 
-// The tile of keys a workgroup takes: the tiles holding keys are dealt to the
-// XCDs in contiguous runs, so that neighbouring tiles, whose counts share
-// lines of hist and whose runs of a digit meet in a line of the output, write
-// them through one L2; the workgroups past them take the rest in order. Dealt
-// round-robin, lines written in parts by several XCDs went to memory in parts:
-// 39M pairs took 248 us a downsweep and 55 us an upsweep (which also wrote the
-// rows of digits the pass does not have), now 201 and 38.
+// The tile of keys a workgroup takes: from kDealTiles tiles on those holding
+// keys are dealt to the XCDs in contiguous runs, so that neighbouring tiles,
+// whose counts share lines of hist and whose runs of a digit meet in a line of
+// the output, write them through one L2; the workgroups past them take the rest
+// in order. Dealt round-robin, lines written in parts by several XCDs went to
+// memory in parts: 39M pairs took 248 us a downsweep and 55 us an upsweep
+// (which also wrote the rows of digits the pass does not have), now 201 and 38.
+// Up to four tiles a CU all run at once, and the runs cost more than they save:
+// six passes over 1M 64-bit keys 123 us round-robin, 141 in runs, over 3M 206
+// and 188.
+constexpr int64_t kDealTiles = 1024;
+
 __device__ __forceinline__ int64_t sort_tile_of(int64_t n, int tile) {
     const int64_t act = (n + tile - 1) / tile, b = blockIdx.x;
-    return b < act ? xcd_contiguous(b, act) : b;
+    return act >= kDealTiles && b < act ? xcd_contiguous(b, act) : b;
 }
 
 template <typename K, int kSortItems>
@@ -132,9 +137,10 @@ __global__ __launch_bounds__(kSortThreads) void radix_upsweep_kernel(const K *ke
 // digit total to totals[d]. Digits the pass does not have (d above its mask)
 // count nothing and are not scanned. A thread takes kScanPer consecutive
 // counts, all requested at once: a count a thread made a chain of 46 dependent
-// round trips over the 11.8k tiles of 48M pairs (30 us a pass, now 17).
-constexpr int kScanPer = 16;
-
+// round trips over the 11.8k tiles of 48M pairs (30 us a pass, now 17). It
+// takes as many as the tiles need for one round, up to 16: with 16 always, six
+// passes over 20k keys took 79 us, with 1 there 74.
+template <int kScanPer>
 __global__ __launch_bounds__(kSortThreads) void radix_scan_kernel(uint32_t *hist, int64_t ntiles,
                                                                   uint32_t *totals, int shift,
                                                                   uint32_t mask,
@@ -399,6 +405,9 @@ int32_t radix_sort_passes(K *keys_in, V *vals_in, K *keys_out, V *vals_out,
     V *src_v = vals_in, *dst_v = vals_out;
     MG_REQUIRE(lo <= hi, "%s: empty key window", who);
     const KeyWin<K> win{lo, hi};
+    const auto scan = ntiles <= kSortThreads       ? radix_scan_kernel<1>
+                      : ntiles <= 4 * kSortThreads ? radix_scan_kernel<4>
+                                                   : radix_scan_kernel<16>;
     TimedScope ts(who, s);
     // Passes of at most 8 bits, the widths as even as the bit count allows
     // (13 bits: 7 + 6, not 8 + 5), so no pass has short digit runs.
@@ -411,8 +420,8 @@ int32_t radix_sort_passes(K *keys_in, V *vals_in, K *keys_out, V *vals_out,
     radix_upsweep_kernel<K, IT><<<(unsigned)ntiles, kSortThreads, 0, s>>>(                 \
         src_k, n, b, mask, win, dw, hist, ntiles, status);                                 \
     MG_LAUNCHED("radix_upsweep_kernel");                                                   \
-    radix_scan_kernel<<<kRadix, kSortThreads, 0, s>>>(hist, ntiles, totals, b, mask,       \
-                                                      dw ? &dw->bits : nullptr);           \
+    scan<<<kRadix, kSortThreads, 0, s>>>(hist, ntiles, totals, b, mask,                    \
+                                         dw ? &dw->bits : nullptr);                        \
     MG_LAUNCHED("radix_scan_kernel");                                                      \
     radix_downsweep_kernel<K, V, IT><<<(unsigned)ntiles, kSortThreads, 0, s>>>(            \
         src_k, src_v, dst_k, dst_v, n, b, mask, win, dw, hist, ntiles, totals, status);    \

@@ -596,6 +596,14 @@ def test_radix_sort_large_tiles(dev, n, bits):
     test_radix_sort_is_stable_and_exact(dev, n, bits)
 
 
+@pytest.mark.parametrize("n", [261_121, 262_143, 262_144, 524_288, 524_289, 2_095_104, 2_095_105,
+                               2_097_152, 2_097_153])
+def test_radix_sort_at_the_edges_of_its_scan_and_dealing(dev, n):
+    """Either side of 256 tiles (of 1024 and of 2048 keys) and of 1024, where
+    the scan's counts a thread and the tiles' order change."""
+    test_radix_sort_is_stable_and_exact(dev, n, (3, 20))
+
+
 @pytest.mark.parametrize("n", [1, 7, 2047, 2048, 2049, 100_003])
 @pytest.mark.parametrize("bits", [(0, 44), (0, 40), (0, 64), (8, 20)])
 def test_radix_sort_is_stable_and_exact(dev, n, bits):
