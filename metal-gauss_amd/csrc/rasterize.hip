@@ -156,27 +156,29 @@ __device__ __forceinline__ float rect_min_q(float mux, float muy, float a, float
     return best;
 }
 
-// One batch entry's record in LDS, 48 bytes: the walks read it with one
-// address as two full 16-byte words and one 4-byte word. With the nine floats
-// in three float4s of which three lanes each were used, the compiler read 12
-// bytes of each, and a 12-byte LDS read takes about twice a 16-byte one's
-// cycles here: the LDS was active 29.4M cycles in the forward's walk at 300k
-// Gaussians and 800x800, now 13.5M (and one address register an entry instead
-// of three).
-struct __align__(16) LdsRec {
-    float4 geo;       // u, v, opacity, red
-    float4 con;       // scaled conic (see scale_conic), green
+// What a batch entry's LDS holds beside its geometry and conic. An entry is
+// three 16-byte words, one in each of three arrays: the walks read two full
+// words and four bytes with one address, 16 j. With three floats in each of
+// three float4s the compiler read 12 bytes of each, and a 12-byte LDS read takes
+// about twice a 16-byte one's cycles here: the LDS was active 29.4M cycles in
+// the forward's walk at 300k Gaussians and 800x800, with full words 13.5M. One
+// record of 48 bytes has an address that takes a multiplication more, in the
+// chain from an entry's index to its math: 10k Gaussians at 256x256 47.3 us in
+// the backward and 58.0 with |d uv|, against 46.3 and 56.1.
+struct __align__(16) LdsRest {
     float blue;
     int32_t id;
     uint32_t live;    // bit w: wave w may be touched
     float pad;
 };
-static_assert(sizeof(LdsRec) == 48, "three 16-byte words");
+static_assert(sizeof(LdsRest) == 16, "one word");
 
 // LDS of one workgroup; MAXW bounds the waves per tile (4 up to 16x16).
 template <int MAXW>
 struct Stage {
-    LdsRec rec[kBatch];
+    float4 geo[kBatch];       // u, v, opacity, red
+    float4 con[kBatch];       // scaled conic (see scale_conic), green
+    LdsRest rest[kBatch];
     uint8_t list[MAXW][kBatch];   // each wave's live entries
     float4 rect[MAXW];            // x_lo, x_hi, y_lo, y_hi of pixel centres
     int32_t flag[MAXW];
@@ -320,10 +322,10 @@ __device__ __forceinline__ Rec gather_rec(const RasterArgs &A, int g) {
 // Writes entry t's record to LDS with its per-wave cull bits.
 template <class S_>
 __device__ __forceinline__ void put_rec(S_ &S, int t, const Rec &r, int nwaves) {
-    S.rec[t].geo = r.geo;
-    S.rec[t].con = scale_conic(r.con);
-    S.rec[t].blue = r.blue;
-    S.rec[t].id = r.id;
+    S.geo[t] = r.geo;
+    S.con[t] = scale_conic(r.con);
+    S.rest[t].blue = r.blue;
+    S.rest[t].id = r.id;
     const float thr = 2.0f * __logf(fmaxf(255.0f * r.geo.z, 1.0f));
     const float thr_m = thr * 1.0001f + 1e-4f;
     uint32_t m = 0;
@@ -335,7 +337,7 @@ __device__ __forceinline__ void put_rec(S_ &S, int t, const Rec &r, int nwaves) 
             rect_min_q(r.geo.x, r.geo.y, ca, r.con.y, cc, ia, ic, q.x, q.y, q.z, q.w) < thr_m)
             m |= 1u << w;
     }
-    S.rec[t].live = m;
+    S.rest[t].live = m;
 }
 
 template <class S_>
@@ -364,7 +366,7 @@ __device__ __forceinline__ int compact_live(S_ &S, int n, int lim, int wave, int
     int cnt = 0;
     for (int c = 0; c < n; c += 64) {
         const int j = c + lane;
-        const bool bit = j < n && j < lim && ((S.rec[j].live >> wave) & 1u);
+        const bool bit = j < n && j < lim && ((S.rest[j].live >> wave) & 1u);
         const uint64_t m = ballot(bit);
         if (bit) S.list[wave][cnt + rank_in(m)] = (uint8_t)j;
         cnt += __popcll(m);
@@ -613,9 +615,9 @@ __global__ __launch_bounds__(MAXW * 64) __attribute__((amdgpu_waves_per_eu(8))) 
                     // below); a scalar min keeps the lane index in scalar registers.
                     const int ku = min(k + u, cnt - 1);
                     jj[u] = __builtin_amdgcn_readlane(lreg, ku & 63);
-                    gg[u] = S.rec[jj[u]].geo;
-                    kk[u] = S.rec[jj[u]].con;
-                    bb[u] = S.rec[jj[u]].blue;
+                    gg[u] = S.geo[jj[u]];
+                    kk[u] = S.con[jj[u]];
+                    bb[u] = S.rest[jj[u]].blue;
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
@@ -875,8 +877,8 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
         float s[kSlots];
 #pragma unroll
         for (int q = 0; q < kSlots; ++q) s[q] = S.grad[q][e];
-        const float op = S.rec[e].geo.z;
-        const float3 con = raw_conic(S.rec[e].con);
+        const float op = S.geo[e].z;
+        const float3 con = raw_conic(S.con[e]);
         S.grad[0][e] = op * fmaf(con.x, s[3], con.y * s[4]);
         S.grad[1][e] = op * fmaf(con.y, s[3], con.z * s[4]);
         S.grad[2][e] = -0.5f * op * s[5];
@@ -895,7 +897,7 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
         for (int idx = (int)threadIdx.x; idx < V * n; idx += (int)blockDim.x) {
             const int e = idx / V, v = idx - V * e;
             const float val = S.grad[v][e];
-            if (val != 0.f) unsafeAtomicAdd(G.rec + (int64_t)kRecFloats * S.rec[e].id + v, val);
+            if (val != 0.f) unsafeAtomicAdd(G.rec + (int64_t)kRecFloats * S.rest[e].id + v, val);
         }
     };
 
@@ -941,8 +943,8 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
             int k = cnt - 1;
             int lreg = S.list[wave][(k & ~63) + lane];
             int ja = __builtin_amdgcn_readlane(lreg, k & 63), jc;
-            float4 geo_a = S.rec[ja].geo, con_a = S.rec[ja].con;
-            float col_a = S.rec[ja].blue;
+            float4 geo_a = S.geo[ja], con_a = S.con[ja];
+            float col_a = S.rest[ja].blue;
             float4 geo_c, con_c;
             float col_c;
             // Entry k - 1 into (jx, x) and entry max(k - 2, 0) into (jy, y).
@@ -951,15 +953,15 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
                 const int kb = k - 1;
                 if ((kb & 63) == 63) lreg = S.list[wave][(kb & ~63) + lane];
                 jx = __builtin_amdgcn_readlane(lreg, kb & 63);
-                gx = S.rec[jx].geo;
-                kx = S.rec[jx].con;
-                cx = S.rec[jx].blue;
+                gx = S.geo[jx];
+                kx = S.con[jx];
+                cx = S.rest[jx].blue;
                 const int kc = max(k - 2, 0);
                 if ((kc & 63) == 63) lreg = S.list[wave][(kc & ~63) + lane];
                 jy = __builtin_amdgcn_readlane(lreg, kc & 63);
-                gy = S.rec[jy].geo;
-                ky = S.rec[jy].con;
-                cy = S.rec[jy].blue;
+                gy = S.geo[jy];
+                ky = S.con[jy];
+                cy = S.rest[jy].blue;
             };
             for (;;) {
                 if (k == 0) {
@@ -993,23 +995,23 @@ __global__ __launch_bounds__(MAXW * 64) void raster_bwd_kernel(const RasterArgs 
             int k = cnt - 1;
             int lreg = S.list[wave][(k & ~63) + lane];
             int ja = __builtin_amdgcn_readlane(lreg, k & 63);
-            float4 geo_a = S.rec[ja].geo, con_a = S.rec[ja].con;
-            float col_a = S.rec[ja].blue;
+            float4 geo_a = S.geo[ja], con_a = S.con[ja];
+            float col_a = S.rest[ja].blue;
             for (;;) {
                 // Entry k - 1 (or k again at the end) into the b registers.
                 const int kb = max(k - 1, 0);
                 if ((kb & 63) == 63) lreg = S.list[wave][(kb & ~63) + lane];
                 const int jb = __builtin_amdgcn_readlane(lreg, kb & 63);
-                const float4 geo_b = S.rec[jb].geo, con_b = S.rec[jb].con;
-                const float col_b = S.rec[jb].blue;
+                const float4 geo_b = S.geo[jb], con_b = S.con[jb];
+                const float col_b = S.rest[jb].blue;
                 entry(ja, base + ja, geo_a, con_a, col_a);
                 if (--k < 0) break;
                 const int kc = max(k - 1, 0);
                 if ((kc & 63) == 63) lreg = S.list[wave][(kc & ~63) + lane];
                 ja = __builtin_amdgcn_readlane(lreg, kc & 63);
-                geo_a = S.rec[ja].geo;
-                con_a = S.rec[ja].con;
-                col_a = S.rec[ja].blue;
+                geo_a = S.geo[ja];
+                con_a = S.con[ja];
+                col_a = S.rest[ja].blue;
                 entry(jb, base + jb, geo_b, con_b, col_b);
                 if (--k < 0) break;
             }
