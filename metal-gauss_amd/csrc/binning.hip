@@ -1037,7 +1037,8 @@ __device__ __forceinline__ void block_excl_sum_max(int vs, int vm, int &ex_s, in
 // Thread k emits the pairs of Gaussian k (tile id key, Gaussian id) at its
 // scanned offset; the workgroup's 256 Gaussians own one contiguous output
 // range.
-//   * Small rectangles (walked by their own thread) go through LDS: their
+//   * Small rectangles (up to kMaskArea tiles; their own thread expands the
+//     count pass's claim mask) go through LDS: their
 //     runs are numbered by a workgroup prefix scan of their counts (at most
 //     256 x 32 pairs) and staged in windows of kBinStage slots, each slot
 //     with its position in the range, then stored by consecutive lanes, so

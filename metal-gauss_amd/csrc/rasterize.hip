@@ -160,9 +160,9 @@ __device__ __forceinline__ float rect_min_q(float mux, float muy, float a, float
 // three 16-byte words, one in each of three arrays: the walks read two full
 // words and four bytes with one address, 16 j. With three floats in each of
 // three float4s the compiler read 12 bytes of each, and a 12-byte LDS read takes
-// about twice a 16-byte one's cycles here: the LDS was active 29.4M cycles in
-// the forward's walk at 300k Gaussians and 800x800, with full words 13.5M. One
-// record of 48 bytes has an address that takes a multiplication more, in the
+// about twice a 16-byte one's cycles here: the LDS was active 37.3M cycles in
+// the forward at 300k Gaussians and 800x800, with full words 17.3M. One record
+// of 48 bytes has an address that takes a multiplication more, in the
 // chain from an entry's index to its math: 10k Gaussians at 256x256 47.3 us in
 // the backward and 58.0 with |d uv|, against 46.3 and 56.1.
 struct __align__(16) LdsRest {
